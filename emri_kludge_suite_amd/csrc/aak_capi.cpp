@@ -352,7 +352,7 @@ static int alloc_lane(aak_handle h, Lane &L) {
   const size_t o_ties = carve(sizeof(FoldTie) * 3 * (size_t)nblk * kFoldMaxTies);
   const size_t o_st = carve(sizeof(int) * 6);
   const size_t o_lw = carve(sizeof(long long) * 2 * 3 * (size_t)nblk * kLW);
-  const size_t o_lc = carve(sizeof(unsigned) * 4);
+  const size_t o_lc = carve(sizeof(unsigned) * 2 * 3 * kLookCtrStride);
   HIPCHK(hipMalloc(&L.d_foldmem, bytes));
   char *base = (char *)L.d_foldmem;
   L.fw.bsum = (double *)(base + o_bsum);
@@ -372,7 +372,7 @@ static int alloc_lane(aak_handle h, Lane &L) {
   L.fw_back = L.fw;
   L.fw_back.status = L.fw.status + 3;
   L.fw_back.look = L.fw.look + 3 * (size_t)nblk * kLW;
-  L.fw_back.look_ctr = L.fw.look_ctr + 1;
+  L.fw_back.look_ctr = L.fw.look_ctr + 3 * kLookCtrStride;
   L.fold_reset = FoldReset{L.fw.look, (int)(2 * 3 * (size_t)nblk * kLW), L.fw.status, L.fw.look_ctr, 0};
   const int nb = h->nbins;
   HIPCHK(hipMalloc(&L.d_hf, sizeof(double2) * 2 * (size_t)nb));

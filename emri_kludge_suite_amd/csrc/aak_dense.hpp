@@ -156,7 +156,8 @@ struct FoldTie {
   long long P;  // inclusive run prefix at the tie (ties rounded down)
 };
 
-constexpr int kLW = 8;  // look-back words per block and phase of the single-pass fold
+constexpr int kLW = 16;  // look-back words per block and phase of the single-pass fold (one 128-byte line)
+constexpr int kLookCtrStride = 32;  // block tickets: one counter per phase, each on a 128-byte line
 
 // What k_guard clears before the folds of a waveform: the look-back words,
 // replay marks and tickets of both fold directions.
@@ -164,7 +165,7 @@ struct FoldReset {
   long long *words;
   int nwords;
   int *status;    // [2][3]
-  unsigned *ctr;  // [2]
+  unsigned *ctr;  // [2][3][kLookCtrStride]
   int force;      // 1: every phase takes the serial replay (test hook)
 };
 
@@ -185,7 +186,7 @@ struct FoldWork {
   FoldTie *ties;                        // [3][nblk][kFoldMaxTies]
   int *status;                          // [3]: 0 ok, 1 overflow/fallback (one fold direction)
   long long *look;                      // [3][nblk][kLW]: look-back words of the single-pass fold
-  unsigned *look_ctr;                   // [1]: block tickets of the single-pass fold
+  unsigned *look_ctr;                   // [3][kLookCtrStride]: block tickets of the single-pass fold
   int *fallbacks;                       // serial replays since the last counter reset
   int force_replay;                     // test hook: 1 every phase takes the serial replay, 2 the middle block fails
 };

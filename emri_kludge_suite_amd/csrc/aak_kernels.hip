@@ -194,15 +194,19 @@ void launch_rates(const DenseParams &P, const DenseBuffers &B, hipStream_t s) {
 constexpr int kGuardThreads = 1024;
 
 // Look-back words of the single-pass fold (k_fold_resolve), kLW per block and
-// phase, reset by k_guard for every waveform: the exact action of a pure
-// block (even and odd start) and its grid key, the exact end value, and the
-// approximate sum and L1 norm of the block's increments and their inclusive
-// prefixes.  "Not yet", "failed" and "not pure" are signalling-NaN patterns
-// that arithmetic never produces and no run total or key can equal.
-constexpr int kLwA0 = 0, kLwA1 = 1, kLwKey = 2, kLwIncl = 3, kLwAggS = 4, kLwAggL = 5, kLwIncS = 6, kLwIncL = 7;
+// phase, reset by k_guard for every waveform: the action of a block on one
+// grid and its grid key, the exact end value, the approximate sum and L1 norm
+// of the block's increments and their inclusive prefixes; then, of a block
+// with a crossing action, its grid keys, its representative start and the
+// four ends (CrossAction).  "Not yet", "failed", "no action" and "crossing"
+// are signalling-NaN patterns that arithmetic never produces and no run total
+// or key can equal.
+constexpr int kLwAct = 0, kLwKey = 2, kLwIncl = 3, kLwAggS = 4, kLwAggL = 5, kLwIncS = 6, kLwIncL = 7;
+constexpr int kLwXKey = 8, kLwXBase = 9, kLwXEnd = 10;  // ends: words 10..13
 constexpr long long kLookEmpty = 0x7FF4A5A5A5A5A5A5LL;
 constexpr long long kLookFail = 0x7FF4A5A5A5A5A5A6LL;
 constexpr long long kLookNone = 0x7FF4A5A5A5A5A5A7LL;
+constexpr long long kLookCross = 0x7FF4A5A5A5A5A5A8LL;
 constexpr int kGuardPer = 32;  // consecutive samples per thread and chunk
 constexpr int kGuardSpinCap = 1 << 22;
 
@@ -214,7 +218,7 @@ __global__ __launch_bounds__(kGuardThreads) void k_guard(DenseParams P, DenseBuf
     const int gt = blockIdx.x * blockDim.x + threadIdx.x, gs = gridDim.x * blockDim.x;
     for (int k = gt; k < R.nwords; k += gs) R.words[k] = kLookEmpty;
     if (R.status && gt < 6) R.status[gt] = R.force == 1 ? 1 : 0;
-    if (R.ctr && gt < 2) R.ctr[gt] = 0;
+    if (R.ctr && gt < 2 * 3 * kLookCtrStride) R.ctr[gt] = 0;
   }
   if (P.guard_last <= P.i0 || B.flags[0] == 0) return;
   __shared__ int s_w[kGuardThreads / 64];
@@ -1018,31 +1022,35 @@ __global__ __launch_bounds__(kChainThreads) void k_fold_chain(FoldArgs A, FoldWo
 }
 
 // Single-pass alternative to k_fold_local<false> + k_fold_chain +
-// k_fold_local<true>: each workgroup classifies its block as above, keeps the
-// item and tie lists in LDS, and obtains the exact value before its first
-// step by a decoupled look-back over the blocks before it (Merrill and
-// Garland, "Single-pass Parallel Prefix Scan with Decoupled Look-back",
-// 2016), with the exact fold as the operator:
-// - a block that is one run on one binade grid without ties ("pure") acts on
-//   the value before it as m -> m + R (m the value in units of its binade's
-//   ulp), so consecutive pure blocks on one grid compose by adding their
-//   totals; it publishes R as soon as it has classified its steps.  Its grid
-//   is that of its first step, which every block can compute from the plan's
-//   approximate block start, so R is published alone;
-// - every block publishes its exact end value after its own serial walk.
+// k_fold_local<true>: each workgroup rounds the increments of its block on
+// the block's grid and obtains the exact value before its first step by a
+// decoupled look-back over the blocks before it (Merrill and Garland,
+// "Single-pass Parallel Prefix Scan with Decoupled Look-back", 2016), with
+// the exact fold as the operator:
+// - a block whose values lie on one binade grid for certain acts on the value
+//   before it as m -> m + R (m the value in units of its binade's ulp), so
+//   consecutive such blocks on one grid compose by adding their totals; it
+//   publishes R and its grid key as soon as it has its approximate start;
+// - a block that crosses into the next binade once, or holds exact ties, acts
+//   on the value before it through that value's last two bits (CrossAction):
+//   it publishes the ends of four representative starts, and later blocks
+//   apply it themselves;
+// - every block publishes its exact end value.
 // Each published value is one 64-bit word written and polled with relaxed
 // device-scope atomics, so no fence orders it against anything else; "not
 // yet" and "failed" are signalling-NaN patterns arithmetic never produces.
 // The look-back reads 64 predecessors at a time with one wave, adds the
-// totals of the nearest run of pure blocks on one grid and stops at the first
-// block with an exact end value; it waits only on blocks that are not pure on
-// that grid.  Every block checks its own start and end against its binades
-// as the chain does, so a result that passes is the chain's result bit for
-// bit; a failed check, an overflowing list or a wait longer than kLookSpinCap
-// polls marks the phase, which k_fold_replay then replays serially.
-// Blocks take tickets from a counter in the order they start, so every block
-// a workgroup waits on has started before it and waits only on earlier
-// blocks itself: the waits cannot form a cycle.
+// totals of the nearest run of blocks on one grid, sets each crossing block it
+// meets aside and stops at the first block with an exact end value, from
+// which it applies them forward; it waits only on blocks that are neither
+// (the first one, and those whose binade the approximate values leave open).
+// Every block checks its own start and end against its binades as the chain
+// does, so a result that passes is the chain's result bit for bit; a failed
+// check, too many serial units or a wait longer than kLookSpinCap polls marks
+// the phase, which k_fold_replay then replays serially.
+// Blocks take tickets from their phase's counter in the order they start, so
+// every block a workgroup waits on has started before it and waits only on
+// earlier blocks itself: the waits cannot form a cycle.
 constexpr int kLookSpinCap = 1 << 18;
 
 __device__ inline long long look_load(const long long *v) {
@@ -1075,49 +1083,86 @@ __device__ inline int exact_key(double x) {
   return (kx + 4096) * 2 + (x > 0.0 ? 1 : 0);
 }
 
-// Look-back state of block j: 2 end value known (or failed), 1 pure with its
-// action published, 0 neither yet (or not pure).  The action of a pure block
-// with ties on its grid depends on the parity of the value before it (each
-// tie rounds to even), so it is published as two totals: a[q] is added to m
-// when m is even (q = 0) or odd (q = 1).  Such actions compose: m -> m +
-// F[m & 1] followed by m -> m + G[m & 1] is m -> m + H[m & 1] with
-// H[q] = F[q] + G[(q + F[q]) & 1].
+// Action of a block whose steps are runs on grid kin, one certain step into
+// the next binade up or down, and runs on grid kout.  Moving the start by 4
+// units of kin's ulp keeps every parity on the way (ties round alike) and
+// moves the end by 2, 4 or 8 units of kout's ulp (one binade up, none, one
+// down), so the ends of four consecutive starts m0 .. m0 + 3 (m0 a multiple
+// of 4) give the end of any other start on grid kin.
+struct CrossAction {
+  int kin, kout;     // binade keys; kin < 0: none
+  long long m0;
+  long long end[4];
+};
+
+// Look-back state of block j: 2 end value known (or failed; v its bits), 1 on
+// one grid with its action published (v the total, key the grid), 3 crossing
+// with its action published, 0 none of these (yet).
 struct LookState {
   int st;
-  long long v;       // st 2: end value bits
-  long long a0, a1;  // st 1: the totals for an even and an odd start
+  long long v;
 };
 __device__ inline LookState look_state(const long long *lw, int j, int &key) {
   const long long *w = lw + (size_t)j * kLW;
   const long long iw = look_load(w + kLwIncl);  // all loads in flight at once
-  const long long w0 = look_load(w + kLwA0), w1 = look_load(w + kLwA1), kw = look_load(w + kLwKey);
+  const long long aw = look_load(w + kLwAct), kw = look_load(w + kLwKey);
   key = -1;
-  if (iw != kLookEmpty) return {2, iw, 0, 0};
-  if (w0 != kLookEmpty && w0 != kLookNone && w1 != kLookEmpty && kw != kLookEmpty) {
+  if (iw != kLookEmpty) return {2, iw};
+  if (aw == kLookCross) return {3, 0};
+  if (aw != kLookEmpty && aw != kLookNone && kw != kLookEmpty) {
     key = (int)kw;
-    return {1, 0, w0, w1};
+    return {1, aw};
   }
-  return {0, 0, 0, 0};
+  return {0, 0};
 }
 
-// (far then near) as one action
-__device__ inline void act_compose(long long f0, long long f1, long long &n0, long long &n1) {
-  const long long h0 = f0 + ((f0 & 1) ? n1 : n0);
-  const long long h1 = f1 + ((f1 & 1) ? n0 : n1);
-  n0 = h0;
-  n1 = h1;
+// The action of crossing block j (state 3).  Its words are stored before the
+// state's, but unordered with it: each is polled until it is there.
+__device__ inline bool cross_load(const long long *lw, int j, CrossAction &c) {
+  const long long *w = lw + (size_t)j * kLW;
+  for (int spins = 0; spins <= kLookSpinCap; spins++) {
+    const long long k = look_load(w + kLwXKey);
+    c.m0 = look_load(w + kLwXBase);
+    bool have = k != kLookEmpty && c.m0 != kLookEmpty;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      c.end[r] = look_load(w + kLwXEnd + r);
+      have = have && c.end[r] != kLookEmpty;
+    }
+    if (have) {
+      c.kin = (int)(k & 0xffffff);
+      c.kout = (int)(k >> 24);
+      return true;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return false;
 }
 
-// The value before a block from an exact end value w and the pure blocks
-// combined after it (key K, action c0/c1; K < 0: none).
-__device__ inline bool look_finish(long long w, int K, long long c0, long long c1, double &x_out) {
+// The end of a crossing block that starts at x; false when x is not on its grid.
+__device__ inline bool cross_apply(const CrossAction &c, double &x) {
+  if (exact_key(x) != c.kin) return false;
+  const int ki = (c.kin >> 1) - 4096, ko = (c.kout >> 1) - 4096;
+  const long long m = (long long)ldexp(x, 53 - ki);
+  const int r = (int)(m & 3);
+  const long long q = (m - c.m0 - r) >> 2;  // exact
+  const long long e = r == 0 ? c.end[0] : r == 1 ? c.end[1] : r == 2 ? c.end[2] : c.end[3];
+  const long long n = e + q * (ko > ki ? 2 : ko == ki ? 4 : 8);
+  const long long an = n < 0 ? -n : n;
+  if (an < (1LL << 52) || an >= (1LL << 53)) return false;
+  x = ldexp((double)n, ko - 53);
+  return true;
+}
+
+// The value before a block from an exact end value w and the blocks combined
+// after it (key K, total c; K < 0: none).
+__device__ inline bool look_finish(long long w, int K, long long c, double &x_out) {
   if (w == kLookFail) return false;
   double x = __longlong_as_double(w);
   if (K >= 0) {
     if (exact_key(x) != K) return false;
     const int k = (K >> 1) - 4096;
-    long long m = (long long)ldexp(x, 53 - k);
-    m += (m & 1) ? c1 : c0;
+    const long long m = (long long)ldexp(x, 53 - k) + c;
     const long long am = m < 0 ? -m : m;
     if (am < (1LL << 52) || am >= (1LL << 53)) return false;
     x = ldexp((double)m, k - 53);
@@ -1126,60 +1171,99 @@ __device__ inline bool look_finish(long long w, int K, long long c0, long long c
   return true;
 }
 
+// One phase of one fold direction: its arrays picked once, at the top of the
+// kernel, so that they stay in scalar registers.
+struct FoldPhase {
+  const double *rate;
+  double *out;
+  double x0, dt;
+  int i0, nsteps;
+};
+
+// Crossing blocks met by one look-back, nearest first, each with the blocks
+// on one grid combined after it.  A waveform's phase crosses a binade about
+// 20 times, most of them inside block 0, which no block looks past; a block
+// beyond the stack's end is waited for.
+constexpr int kLookStack = 32;
+struct LookPending {
+  long long c;
+  int K, j;
+};
+
 // Wave 0: exact value before block b's first step.  Returns false when the
 // phase failed (a failed predecessor, a failed binade check, a wait past the
-// cap).
-__device__ inline bool fold_look_back(const FoldArgs &A, const long long *lw, int p, int b, double &x_out) {
+// cap).  `pend`: kLookStack entries of LDS.
+__device__ inline bool fold_look_back(const FoldPhase &F, const long long *lw, int b, LookPending *pend,
+                                      double &x_out) {
   const int lane = threadIdx.x & 63;
-  int j = b - 1;              // nearest block not yet combined
-  int K = -1;                 // binade key of the combined pure blocks
-  long long c0 = 0, c1 = 0;   // their combined action
-  int spins = 0;
+  int j = b - 1;     // nearest block of the window
+  int K = -1;        // grid key of the combined blocks
+  long long c = 0;   // their total
+  int spins = 0, np = 0;
+  // the end value w of a block, through the combined blocks and those set aside
+  auto finish = [&](long long w) {
+    if (!look_finish(w, K, c, x_out)) return false;
+    while (np > 0) {
+      np--;
+      const LookPending &q = pend[np];
+      CrossAction ca;
+      if (!cross_load(lw, q.j, ca) || !cross_apply(ca, x_out)) return false;
+      if (!look_finish(__double_as_longlong(x_out), q.K, q.c, x_out)) return false;
+    }
+    return true;
+  };
   for (;;) {
     const int jb = j - lane;
     // block -1 stands for the start value x0
-    LookState S = {2, __double_as_longlong(A.x0[p]), 0, 0};
+    LookState S = {2, __double_as_longlong(F.x0)};
     int key = -1;
     if (jb >= 0) S = look_state(lw, jb, key);
-    const int s0 = __shfl(S.st, 0, 64);
-    const int k0 = __shfl(key, 0, 64);
-    const int Kc = (K >= 0) ? K : (s0 == 1 ? k0 : -2);
-    const bool ext = S.st == 1 && key == Kc && key >= 0;
-    const unsigned long long mask = __ballot(ext);
-    const int s = (~mask) ? __builtin_ctzll(~mask) : 64;
-    // ordered composition of lanes 0..s-1 (lane 0 nearest): after the step
-    // with offset o, lane l (a multiple of 2o) holds lanes l..l+2o-1
-    long long n0 = (lane < s) ? S.a0 : 0, n1 = (lane < s) ? S.a1 : 0;
+    int start = 0;  // lanes before it are combined or set aside
+    for (;;) {
+      const int s0 = __shfl(S.st, start, 64);
+      const int k0 = __shfl(key, start, 64);
+      const int Kc = (K >= 0) ? K : (s0 == 1 ? k0 : -2);
+      const bool ext = S.st == 1 && key == Kc && key >= 0;
+      const unsigned long long mask = ~(__ballot(ext) >> start);
+      const int s = min(64, mask ? start + __builtin_ctzll(mask) : 64);
+      if (s > start) {
+        long long v = (lane >= start && lane < s) ? S.v : 0;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const long long f0 = __shfl_down(n0, o, 64), f1 = __shfl_down(n1, o, 64);
-      if (lane + o < 64) act_compose(f0, f1, n0, n1);
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        c += v;
+        K = Kc;
+      }
+      if (s == 64) {
+        j -= 64;
+        break;
+      }
+      const int js = j - s, ss = __shfl(S.st, s, 64);
+      if (ss == 2) return finish(__shfl(S.v, s, 64));
+      if (ss == 3 && np < kLookStack) {
+        if (lane == 0) pend[np] = LookPending{c, K, js};
+        __builtin_amdgcn_wave_barrier();
+        np++;
+        K = -1;
+        c = 0;
+        start = s + 1;
+        if (start < 64) continue;
+        j -= 64;
+        break;
+      }
+      // not yet published, or on another grid: wait for a change of state; an
+      // end value is used at once, a newly published action is combined by the
+      // next window, which starts at that block
+      LookState T;
+      int tk;
+      do {
+        if (++spins > kLookSpinCap) return false;
+        __builtin_amdgcn_s_sleep(1);
+        T = look_state(lw, js, tk);
+      } while (T.st == ss);
+      if (T.st == 2) return finish(T.v);
+      j = js;
+      break;
     }
-    {
-      // the window lies before the blocks combined so far
-      long long w0 = __shfl(n0, 0, 64), w1 = __shfl(n1, 0, 64);
-      act_compose(w0, w1, c0, c1);
-    }
-    if (s > 0) K = Kc;
-    if (s == 64) {
-      j -= 64;
-      continue;
-    }
-    const int js = j - s;
-    const int ss = __shfl(S.st, s, 64);
-    if (ss == 2) return look_finish(__shfl(S.v, s, 64), K, c0, c1, x_out);
-    // not yet published, or pure on another grid: wait for a change of state;
-    // an end value is used at once, a newly published action is combined by
-    // the next window, which starts at that block
-    LookState T;
-    int tk;
-    do {
-      if (++spins > kLookSpinCap) return false;
-      __builtin_amdgcn_s_sleep(1);
-      T = look_state(lw, js, tk);
-    } while (T.st == ss);
-    if (T.st == 2) return look_finish(T.v, K, c0, c1, x_out);
-    j = js;
   }
 }
 
@@ -1189,7 +1273,7 @@ __device__ inline bool fold_look_back(const FoldArgs &A, const long long *lw, in
 // the walk back.  The blocks waited on publish their sums without waiting
 // themselves, so the waits are short.  Returns false after a wait past the
 // cap.
-__device__ inline bool approx_look_back(const FoldArgs &A, const long long *lw, int p, int b, double &S, double &L) {
+__device__ inline bool approx_look_back(const FoldPhase &F, const long long *lw, int b, double &S, double &L) {
   const int lane = threadIdx.x & 63;
   int j = b - 1;
   double s = 0.0, l = 0.0;
@@ -1197,7 +1281,7 @@ __device__ inline bool approx_look_back(const FoldArgs &A, const long long *lw, 
   for (;;) {
     const int jb = j - lane;
     int st = 2;  // block -1 stands for the start value
-    double vs = A.x0[p], vl = fabs(A.x0[p]);
+    double vs = F.x0, vl = fabs(F.x0);
     if (jb >= 0) {
       const long long *w = lw + (size_t)jb * kLW;
       const long long is = look_load(w + kLwIncS), il = look_load(w + kLwIncL);
@@ -1245,326 +1329,461 @@ __device__ inline bool approx_look_back(const FoldArgs &A, const long long *lw, 
   }
 }
 
+// Inclusive sum over the wave, lanes in order, by data-parallel moves (shifts
+// inside rows of 16 lanes, then two row broadcasts).
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ inline double wave_scan(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1
+  v = dpp_add<0x112, 0xf>(v);  // row_shr 2
+  v = dpp_add<0x114, 0xf>(v);  // row_shr 4
+  v = dpp_add<0x118, 0xf>(v);  // row_shr 8
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+__device__ inline double lane_readd(double v, int q) { return __longlong_as_double(lane_read64(__double_as_longlong(v), q)); }
+
+// A block's steps in units of 64: register q of wave w holds unit 4 q + w, one
+// step per lane, so loads, stores and scans all run along the lanes.
+constexpr int kFoldUnits = kFoldBlock / 64;
+constexpr int kFoldSerial = 24;  // units of one block that may be replayed step by step
+constexpr int kFoldBatch = 4;     // steps per lane whose loads are in flight together
+static_assert(kFoldUnits == 64, "one lane per unit");
+
+// Place of step `off` of a block among its 4096 array elements, lowest index first.
 template <int DIR>
-__global__ __launch_bounds__(kFoldThreads, 3) void k_fold_resolve(FoldArgs A, FoldWork W) {
-  __shared__ double shd[kFoldThreads / 64];
-  __shared__ long long shl[2 * (kFoldThreads / 64)];
-  __shared__ int shi[kFoldThreads];
-  __shared__ int shf[kFoldThreads / 64];
-  __shared__ double sd[kFoldLds];
-  __shared__ FoldItem s_items[kFoldMaxItems];
-  __shared__ FoldTie s_ties[kFoldMaxTies];
-  __shared__ double s_x[kFoldMaxItems];
-  __shared__ double s_xs, s_E;
-  __shared__ int s_pb[2], s_ok;
-  const int tid = threadIdx.x;
+__device__ inline unsigned fold_elem(unsigned off) { return DIR > 0 ? off : kFoldBlock - 1 - off; }
+
+// The increments of block b, through a buffer descriptor of its elements (one
+// offset register for all loads); steps past the end read the last step's
+// rates (in bounds).
+template <int DIR>
+__device__ inline void load_increments(const FoldPhase &F, int b, double *d) {
+  const int ib = F.i0 + DIR * b * kFoldBlock;
+  const unsigned n = (unsigned)min(kFoldBlock, F.nsteps - b * kFoldBlock);
+  const double *base = F.rate + (DIR > 0 ? ib : ib - (kFoldBlock - 1));
+  const double *prev = b > 0 ? base - DIR : base;  // the rate of the step before; step 0 takes its own
+  const int shift = b > 0 ? 0 : -8 * DIR;
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  const auto rb = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, kFoldBlock * 8, 0x00020000);
+  const auto rp = __builtin_amdgcn_make_buffer_rsrc((void *)prev, 0, kFoldBlock * 8, 0x00020000);
+  unsigned tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // offsets are cheaper formed again than kept
+#pragma unroll
+  for (int h = 0; h < kFoldPerThread; h += kFoldBatch) {
+    double r[kFoldBatch], rm[kFoldBatch];
+#pragma unroll
+    for (int q = 0; q < kFoldBatch; q++) {
+      const int e = 8 * (int)fold_elem<DIR>(min(tid + (h + q) * kFoldThreads, n - 1));
+      r[q] = __builtin_bit_cast(double, (v2i)__builtin_amdgcn_raw_buffer_load_b64(rb, e, 0, 0));
+      // step 0 of the fold reads out of the descriptor's range (0) and is set below
+      rm[q] = __builtin_bit_cast(double, (v2i)__builtin_amdgcn_raw_buffer_load_b64(rp, e + shift, 0, 0));
+    }
+#pragma unroll
+    for (int q = 0; q < kFoldBatch; q++) {
+      if (h + q == 0 && b == 0 && tid == 0) rm[q] = r[q];
+      const double v = (1.5 * r[q] - .5 * rm[q]) * F.dt;
+      d[h + q] = (tid + (h + q) * kFoldThreads < n) ? (DIR > 0 ? v : -v) : 0.0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Grid of the values on the way from a through increments of sum s and L1 norm
+// l, each known to within E, where that is certain: the values lie between
+// a - (l - s) / 2 and a + (l + s) / 2.  The frexp exponent, or -5000; also
+// -5000 where an increment may pass a quarter of the binade (the rounding by
+// 1.5 2^52 u needs |d| <= 2^51 u).
+__device__ inline int sure_exponent(double a, double s, double l, double E) {
+  double lo = a - 0.5 * (l - s), hi = a + 0.5 * (l + s);
+  if (a < 0.0) {
+    const double t = lo;
+    lo = -hi;
+    hi = -t;
+  }
+  lo -= E;
+  hi += E;
+  if (!(lo > 0.0) || !(hi < 1e300)) return -5000;
+  int k, kh;
+  frexp(lo, &k);
+  frexp(hi, &kh);
+  return k == kh && l < ldexp(0.25, k) ? k : -5000;
+}
+
+// LDS of one workgroup of the single-pass fold.
+struct FoldShared {
+  double red[2 * (kFoldThreads / 64)];
+  double xs, E, x;
+  int t, ok, nserial, unsure;
+  double sum[kFoldUnits], l1[kFoldUnits];  // per unit: approximate sum and L1 norm; rounded total in sum
+  double xu[kFoldUnits];                   // exact start of each unit
+  int slot[kFoldUnits];                    // row of ser holding the unit's increments; -1 on one grid, -2 with ties
+  double adj[kFoldUnits][2];               // of a unit with ties, by parity of its start: what they add to its total
+  unsigned long long flip[kFoldUnits][2];  // and the ties that round the other way
+  unsigned long long up[kFoldUnits];       // ties whose other neighbour lies above
+  double ser[kFoldSerial][64];
+  double park[kFoldPerThread][64];
+  LookPending pend[kLookStack];
+};
+
+// Walk of wave 0 over its block's units from x (EXACT: the same in every lane;
+// otherwise one start per lane).  Lane u holds unit u: its grid exponent,
+// rounded total and serial row.  A run of units on one grid is one add of
+// exact sums; a serial unit is replayed step by step.  EXACT: xu receives the
+// exact start of the lane's unit and the serial units' values are written.
+template <bool EXACT, int DIR>
+__device__ inline bool fold_walk(const FoldPhase &F, FoldShared &S, int b, int k, int slot, double R,
+                                 double &x, double &xu) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long serial = __ballot(slot >= 0), tied = __ballot(slot == -2);
+  bool good = true;
+  int pos = 0;
+  while (pos < kFoldUnits) {
+    const unsigned long long rest = serial >> pos;
+    if (rest & 1) {
+      // a chain of dependent adds, the next increments loaded ahead; EXACT: one
+      // lane walks and leaves each value in its increment's place
+      double *ser = S.ser[__builtin_amdgcn_readlane(slot, pos)];
+      if (!EXACT || lane == 0) {
+        double v[4], w[4];
+        auto chain = [&](int h, double *c) {
+#pragma unroll
+          for (int s = 0; s < 4; s++) c[s] = x = x + c[s];
+          if (EXACT)
+#pragma unroll
+            for (int s = 0; s < 4; s++) ser[h + s] = c[s];
+        };
+#pragma unroll
+        for (int s = 0; s < 4; s++) v[s] = ser[s];
+#pragma unroll 1
+        for (int h = 0; h < 64; h += 8) {
+#pragma unroll
+          for (int s = 0; s < 4; s++) w[s] = ser[h + 4 + s];
+          __builtin_amdgcn_sched_barrier(0);
+          chain(h, v);
+#pragma unroll
+          for (int s = 0; s < 4; s++) v[s] = ser[((h + 8) & 63) + s];
+          __builtin_amdgcn_sched_barrier(0);
+          chain(h + 4, w);
+        }
+      }
+      if (EXACT) {
+        x = uniform_double(x);
+        __builtin_amdgcn_wave_barrier();
+        const int s = b * kFoldBlock + pos * 64 + lane;
+        if (s < F.nsteps) F.out[F.i0 + DIR * (s + 1)] = ser[lane];
+      }
+      pos++;
+      continue;
+    }
+    const int kk = __builtin_amdgcn_readlane(k, pos);
+    const int key = (kk + 4096) * 2 + (x > 0.0 ? 1 : 0);
+    if ((tied >> pos) & 1) {
+      // exact ties: the total by the parity of the start
+      good = good && exact_key(x) == key;
+      if (EXACT && lane == pos) xu = x;
+      x = x + (lane_readd(R, pos) + S.adj[pos][(long long)ldexp(x, 53 - kk) & 1]);
+      good = good && exact_key(x) == key;
+      pos++;
+      continue;
+    }
+    const unsigned long long stop = rest | (tied >> pos);
+    const int end = stop ? pos + __builtin_ctzll(stop) : kFoldUnits;
+    const bool in = lane >= pos && lane < end;
+    good = good && __ballot(in && k != kk) == 0 && exact_key(x) == key;
+    const double incl = wave_scan(in ? R : 0.0);
+    if (EXACT && in) xu = x + (incl - R);
+    x = x + lane_readd(incl, 63);
+    good = good && exact_key(x) == key;
+    pos = end;
+  }
+  return good;
+}
+
+// The kernel is bound by latency: a block loads, waits for the approximate
+// sums of those before it, rounds, and waits for its exact start.  So what
+// counts is that all blocks of a 2^21-sample waveform run at once (1536
+// workgroups; six per CU) and that no block is late.  A block on one grid u
+// (all but about 20 per phase) rounds each step with one add and one subtract
+// of 1.5 2^52 u, and every sum of the rounded steps is a multiple of u below
+// 2^53 u, so plain FP64 scans are exact; its steps stay in registers, one
+// per lane, from load to store.  Other blocks test each unit of 64 steps in
+// the same way and replay the few units that hold a crossing or a tie.
+// Classifying every step into item lists staged in LDS (39 KB, four
+// workgroups per CU, a second wave of them) took 78 us per waveform at
+// N = 2^21, this form 61 us.
+template <int DIR>
+__global__ __launch_bounds__(kFoldThreads, 6) void k_fold_resolve(FoldArgs A, FoldWork W) {
+  __shared__ FoldShared S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int p = blockIdx.y;
+  const FoldPhase F = {A.rate[p], A.out[p], A.x0[p], A.dt, A.i0, A.nsteps};
+  int *status = W.status + p;
+  unsigned *ctr = W.look_ctr + p * kLookCtrStride;
+  long long *lw = W.look + (size_t)p * A.nblk * kLW;
   if (tid == 0) {
-    const unsigned t = atomicAdd(W.look_ctr, 1u);
-    s_pb[0] = (int)(t % 3u);
-    s_pb[1] = (int)(t / 3u);
+    S.t = (int)atomicAdd(ctr, 1u);
+    S.nserial = 0;
+    S.unsure = 0;
+    // entry: a phase already marked (the replay hook) skips to the end
+    S.ok = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
   }
   __syncthreads();
-  const int p = __builtin_amdgcn_readfirstlane(s_pb[0]), b = __builtin_amdgcn_readfirstlane(s_pb[1]);
-  long long *lw = W.look + (size_t)p * A.nblk * kLW;
+  const int b = __builtin_amdgcn_readfirstlane(S.t);
   long long *mw = lw + (size_t)b * kLW;  // this block's words
-  // entry: a phase already marked (the replay hook) skips to the end
-  if (tid == 0) s_ok = __hip_atomic_load(W.status + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-  __syncthreads();
-  bool ok = s_ok != 0;
-  const int base = b * kFoldBlock + tid * kFoldPerThread;
   double d[kFoldPerThread];
-  int key[kFoldPerThread];
-  long long r[kFoldPerThread];
-  int tie_mask = 0, head_mask = 0;
-  bool next_starts = true;
-  long long carry = 0;
-  int item_base = 0, tie_base = 0;
-  // the increments, and the block's approximate sum and L1 norm, published at
-  // once for the approximate look-back of the blocks after it
-  stage_increments<DIR>(A, p, b, sd);
+  load_increments<DIR>(F, b, d);
+  // the block's approximate sum and L1 norm, published at once for the
+  // approximate look-back of the blocks after it
   double tsum = 0.0, tl1 = 0.0;
 #pragma unroll
-  for (int j = 0; j < kFoldPerThread; j++) {
-    const double v = sd[fold_lds_index(tid * kFoldPerThread + j)];
-    tsum += v;
-    tl1 += fabs(v);
+  for (int q = 0; q < kFoldPerThread; q++) {
+    tsum += d[q];
+    tl1 += fabs(d[q]);
   }
-  double bsum, bl1;
-  const double excl = block_excl_sum(tsum, shd, &bsum);
-  (void)block_excl_sum(tl1, shd, &bl1);
-  if (tid == 0) {
-    look_store(mw + kLwAggL, __double_as_longlong(bl1));
-    look_store(mw + kLwAggS, __double_as_longlong(bsum));
+  tsum = wave_scan(tsum);
+  tl1 = wave_scan(tl1);
+  if (lane == 63) {
+    S.red[wave] = tsum;
+    S.red[kFoldThreads / 64 + wave] = tl1;
+  }
+  __syncthreads();
+  double bsum = 0.0, bl1 = 0.0;
+#pragma unroll
+  for (int w = 0; w < kFoldThreads / 64; w++) {
+    bsum += S.red[w];
+    bl1 += S.red[kFoldThreads / 64 + w];
   }
   // approximate start of the block, and the bound E on the distance between
   // approximate and exact values in it: every value up to the block's end,
   // either way, is at most U = |x0| + the L1 norm so far in magnitude, so
   // each of at most nsteps + 2 kFoldBlock roundings on either path is at most
   // half an ulp of U
-  if (tid < 64) {
-    double S = A.x0[p], L = fabs(A.x0[p]);
-    const bool aok = (b == 0) || approx_look_back(A, lw, p, b, S, L);
-    if (tid == 0) {
+  if (wave == 0) {
+    if (lane == 0) {
+      look_store(mw + kLwAggL, __double_as_longlong(bl1));
+      look_store(mw + kLwAggS, __double_as_longlong(bsum));
+    }
+    double s = F.x0, L = fabs(F.x0);
+    const bool aok = (b == 0) || approx_look_back(F, lw, b, s, L);
+    if (lane == 0) {
       look_store(mw + kLwIncL, __double_as_longlong(L + bl1));
-      look_store(mw + kLwIncS, __double_as_longlong(S + bsum));
+      look_store(mw + kLwIncS, __double_as_longlong(s + bsum));
       const double U = (L + bl1) * (1.0 + 0x1p-24);
       int ex = 0;
       frexp(U > 0.0 ? U : 1.0, &ex);
-      s_xs = S;
-      s_E = ((double)A.nsteps + 2.0 * kFoldBlock) * ldexp(1.0, ex - 52);
-      if (!aok) s_ok = 0;
+      S.xs = s;
+      S.E = ((double)F.nsteps + 2.0 * kFoldBlock) * ldexp(1.0, ex - 52);
+      if (!aok) S.ok = 0;
     }
   }
   __syncthreads();
-  ok = ok && s_ok != 0;
-  const double E = uniform_double(s_E);
-  if (ok) {
-    // the increments again from LDS (not held across the look-back)
+  const double E = uniform_double(S.E), xs = uniform_double(S.xs);
+  bool ok = __builtin_amdgcn_readfirstlane(S.ok) != 0;
+  const int kb = ok ? __builtin_amdgcn_readfirstlane(sure_exponent(xs, uniform_double(bsum), uniform_double(bl1), E)) : -5000;
+  bool on_grid = kb > -5000;
+  // The loops over the units are rolled and rotate the units through d[0]: the
+  // kernel is short enough for instruction fetch to count.
+  // Wave 0 leaves its steps in LDS while it looks back, so that the look-back's
+  // registers come on top of none of them (80 in all: six workgroups per CU).
+  auto park = [&]() {
 #pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) d[j] = sd[fold_lds_index(tid * kFoldPerThread + j)];
-    double a0 = uniform_double(s_xs) + excl;
-    // keys: >= 0 binade grid, -1 exact replay, -2 beyond the end
+    for (int q = 0; q < kFoldPerThread; q++) S.park[q][lane] = d[q];
+  };
+  auto unpark = [&]() {
 #pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) {
-      const int s = base + j;
-      if (s >= A.nsteps) {
-        key[j] = -2;
-        r[j] = 0;
-        continue;
-      }
-      const double a1 = a0 + d[j];
-      const int k0 = binade_key(a0, E);
-      const int k1 = binade_key(a1, E);
-      if (k0 >= 0 && k0 == k1) {
-        key[j] = k0;
-        const int kexp = (k0 >> 1) - 4096;
-        const double f = ldexp(d[j], 53 - kexp);
-        const double fl = floor(f);
-        const double fr = f - fl;
-        long long ri = (long long)fl;
-        if (fr > 0.5) ri += 1;
-        else if (fr == 0.5) tie_mask |= (1 << j);
-        r[j] = ri;
-      } else {
-        key[j] = -1;
-        r[j] = 0;
-      }
-      a0 = a1;
-    }
-    shi[tid] = key[kFoldPerThread - 1];
-    __syncthreads();
-    const int prev_key = (tid > 0) ? shi[tid - 1] : -3;
-    __syncthreads();
+    for (int q = 0; q < kFoldPerThread; q++) d[q] = S.park[q][lane];
+  };
+  auto rotate = [&](double last) {
 #pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) {
-      const int kprev = (j == 0) ? prev_key : key[j - 1];
-      const bool h = (key[j] != -2) && (key[j] == -1 || kprev == -1 || kprev == -3 || key[j] != kprev);
-      if (h) head_mask |= (1 << j);
-    }
-    shi[tid] = ((head_mask & 1) || key[0] == -2) ? 1 : 0;
-    __syncthreads();
-    next_starts = (tid + 1 < kFoldThreads) ? (shi[tid + 1] != 0) : true;
-    __syncthreads();
-    long long tail = 0;
-    int has_head = 0;
-#pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) {
-      if (head_mask & (1 << j)) {
-        has_head = 1;
-        tail = 0;
-      }
-      tail += r[j];
-    }
-    const long long seg_incl = block_seg_incl(tail, has_head, shl, shf);
-    carry = __shfl_up(seg_incl, 1, 64);
-    if ((tid & 63) == 63) shl[kFoldThreads / 64 + (tid >> 6)] = seg_incl;
-    __syncthreads();
-    if ((tid & 63) == 0) carry = (tid > 0) ? shl[kFoldThreads / 64 + (tid >> 6) - 1] : 0;
-    __syncthreads();
-    int nheads_tot, nties_tot;
-    item_base = block_excl_sum((int)__popc(head_mask), shi, &nheads_tot);
-    tie_base = block_excl_sum((int)__popc(tie_mask), shi, &nties_tot);
-    if (nheads_tot > kFoldMaxItems || nties_tot > kFoldMaxTies) ok = false;
-    if (ok) {
-      // the block's item and tie lists, in LDS
-      long long P = carry;
-      int item = item_base - 1, tcount = tie_base;
-#pragma unroll
-      for (int j = 0; j < kFoldPerThread; j++) {
-        if (key[j] == -2) break;
-        const int sl = tid * kFoldPerThread + j;
-        if (head_mask & (1 << j)) {
-          item++;
-          P = 0;
-          s_items[item].kind = (key[j] == -1) ? 1 : 0;
-          s_items[item].k = (key[j] >= 0) ? (key[j] >> 1) - 4096 : 0;
-          s_items[item].sgn = (key[j] >= 0) ? ((key[j] & 1) ? 1 : -1) : 0;
-          s_items[item].first = sl;
-          s_items[item].tie_first = tcount;
-        }
-        P += r[j];
-        const bool last_of_run = (key[j] >= 0) && ((j + 1 < kFoldPerThread)
-                                                       ? (((head_mask >> (j + 1)) & 1) || key[j + 1] == -2)
-                                                       : next_starts);
-        if (tie_mask & (1 << j)) {
-          s_ties[tcount].step = sl;
-          s_ties[tcount].P = P;
-          s_ties[tcount].up = 0;
-          tcount++;
-        }
-        if (last_of_run) s_items[item].R = P;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      s_pb[0] = nheads_tot;
-      s_pb[1] = nties_tot;
-      // a block that is one run publishes its action at once: the run total
-      // plus the ties rounded up, for an even and for an odd start, and its
-      // grid key
-      const bool pure = ok && nheads_tot == 1 && s_items[0].kind == 0;
-      long long a0 = kLookNone, a1 = kLookNone;
-      if (pure) {
-        long long u0 = 0, u1 = 0;
-        for (int t = 0; t < nties_tot; t++) {
-          const long long P = s_ties[t].P;
-          u0 += (P + u0) & 1;
-          u1 += (1 + P + u1) & 1;
-        }
-        a0 = s_items[0].R + u0;
-        a1 = s_items[0].R + u1;
-      }
-      if (pure) look_store(mw + kLwKey, (long long)((s_items[0].k + 4096) * 2 + (s_items[0].sgn > 0 ? 1 : 0)));
-      look_store(mw + kLwA1, a1);
-      look_store(mw + kLwA0, a0);
-    }
-    __syncthreads();
-  }
-  // wave 0: look back, then the block's own walk; publishes the end value.
-  // Lane q holds item q, with its action on an even and an odd start (its
-  // ties round to even), so the walk reads uniform values from registers and
-  // the end value is published before the ties are resolved for the write.
-  if (tid < 64) {
-    const int lane = tid, ni = ok ? s_pb[0] : 0, nt = ok ? s_pb[1] : 0;
-    int it_kind = 1, it_k = 0, it_sgn = 0, it_t0 = 0, it_t1 = 0;
-    long long it_d = 0, it_a0 = 0, it_a1 = 0;
-    if (lane < ni) {
-      const FoldItem &I = s_items[lane];
-      it_kind = I.kind;
-      it_k = I.k;
-      it_sgn = I.sgn;
-      // a single step's increment, from the staged increments (sd holds them
-      // until the write)
-      it_d = __double_as_longlong(sd[fold_lds_index(I.first)]);
-      if (I.kind == 0) {
-        it_t0 = I.tie_first;
-        it_t1 = (lane + 1 < ni) ? s_items[lane + 1].tie_first : nt;
-        long long u0 = 0, u1 = 0;
-        for (int t = it_t0; t < it_t1; t++) {
-          const long long P = s_ties[t].P;
-          u0 += (P + u0) & 1;
-          u1 += (1 + P + u1) & 1;
-        }
-        it_a0 = I.R + u0;
-        it_a1 = I.R + u1;
-      }
-    }
-    double x = 0.0;
-    bool wok = ok && (b == 0 ? (x = A.x0[p], true) : fold_look_back(A, lw, p, b, x));
-    if (W.force_replay == 2 && b == A.nblk / 2) wok = false;  // test hook
-    if (wok && b == 0 && lane == 0) A.out[p][A.i0] = x;
-    long long my_m = 0;
-    double my_x = 0.0;
-    for (int q = 0; wok && q < ni; q++) {
-      const int kind = __builtin_amdgcn_readlane(it_kind, q);
-      if (kind == 1) {
-        x = x + __longlong_as_double(lane_read64(it_d, q));
-        if (lane == q) my_x = x;
-        continue;
-      }
-      const int k = __builtin_amdgcn_readlane(it_k, q), sgn = __builtin_amdgcn_readlane(it_sgn, q);
-      int kx;
-      frexp(x, &kx);
-      if (kx != k || (x > 0.0 ? 1 : -1) != sgn) {
-        wok = false;
-        break;
-      }
-      long long m = (long long)ldexp(x, 53 - k);
-      if (lane == q) my_m = m;
-      m += (m & 1) ? lane_read64(it_a1, q) : lane_read64(it_a0, q);
-      const long long am = m < 0 ? -m : m;
-      if (am < (1LL << 52) || am >= (1LL << 53)) {
-        wok = false;
-        break;
-      }
-      x = ldexp((double)m, k - 53);
-    }
-    if (wok && !(x == x)) wok = false;  // a NaN phase takes the serial replay
-    if (lane == 0) {
-      if (wok) {
-        look_store(mw + kLwIncl, __double_as_longlong(x));
-      } else {
-        __hip_atomic_store(W.status + p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        look_store(mw + kLwIncl, kLookFail);
-      }
-      s_ok = wok ? 1 : 0;
-    }
-    if (wok && lane < ni) {
-      // exact start of each run and the rounding of its ties, for the write
-      if (it_kind == 1) {
-        s_x[lane] = my_x;
-      } else {
-        s_items[lane].m_start = my_m;
-        long long ups = 0;
-        for (int t = it_t0; t < it_t1; t++) {
-          const int up = (int)((my_m + s_ties[t].P + ups) & 1LL);
-          s_ties[t].up = up;
-          ups += up;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  if (s_ok) {
-    // exact values of every step: runs from their exact starts, single steps
-    // from the walk; staged in LDS and stored coalesced
-    long long P = carry;
-    int item = item_base - 1, tcount = tie_base;
-    int c_item = -1, c_k = 0, c_tf = 0;
-    long long c_m = 0;
-    double outv[kFoldPerThread];
-#pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) {
-      outv[j] = 0.0;
-      if (key[j] == -2) continue;
-      if (head_mask & (1 << j)) {
-        item++;
-        P = 0;
-      }
-      P += r[j];
-      if (tie_mask & (1 << j)) tcount++;
-      if (key[j] >= 0) {
-        if (item != c_item) {
-          c_item = item;
-          c_m = s_items[item].m_start;
-          c_k = s_items[item].k;
-          c_tf = s_items[item].tie_first;
-        }
-        long long ups = 0;
-        for (int q = c_tf; q < tcount; q++) ups += s_ties[q].up;
-        outv[j] = ldexp((double)(c_m + P + ups), c_k - 53);
-      } else {
-        outv[j] = s_x[item];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kFoldPerThread; j++) sd[fold_lds_index(tid * kFoldPerThread + j)] = outv[j];
-    __syncthreads();
-    double *op = A.out[p] + (A.i0 + DIR * (b * kFoldBlock + tid + 1));
-#pragma unroll
+    for (int q = 0; q + 1 < kFoldPerThread; q++) d[q] = d[q + 1];
+    d[kFoldPerThread - 1] = last;
+  };
+  if (on_grid) {
+    const double C = ldexp(1.5, kb - 1), half = ldexp(0.5, kb - 53);
+    int tie = 0;
+#pragma unroll 1
     for (int q = 0; q < kFoldPerThread; q++) {
-      const int s = b * kFoldBlock + tid + q * kFoldThreads;
-      if (s < A.nsteps) op[DIR * q * kFoldThreads] = sd[fold_lds_index(tid + q * kFoldThreads)];
+      const double v = (d[0] + C) - C;
+      tie |= fabs(d[0] - v) == half;
+      const double sc = wave_scan(v);
+      if (lane == 63) S.sum[4 * q + wave] = sc;
+      rotate(sc);
+    }
+    on_grid = __syncthreads_or(tie) == 0;
+    if (!on_grid) load_increments<DIR>(F, b, d);
+  }
+  const int ib = F.i0 + DIR * b * kFoldBlock;
+  double *op = F.out + (DIR > 0 ? ib + 1 : ib - kFoldBlock);  // element 0 of the block
+  const unsigned n = (unsigned)min(kFoldBlock, F.nsteps - b * kFoldBlock);
+  unsigned off0 = tid;
+  asm volatile("" : "+v"(off0));
+  if (on_grid) {
+    const double R = S.sum[lane], incl = wave_scan(R);
+    const double tot = lane_readd(incl, 63);
+    if (wave == 0) {
+      park();
+      const int key = (kb + 4096) * 2 + (xs > 0.0 ? 1 : 0);
+      if (lane == 0) {
+        look_store(mw + kLwKey, (long long)key);
+        look_store(mw + kLwAct, (long long)ldexp(tot, 53 - kb));
+      }
+      double x = 0.0;
+      bool wok = b == 0 ? (x = F.x0, true) : fold_look_back(F, lw, b, S.pend, x);
+      if (W.force_replay == 2 && b == A.nblk / 2) wok = false;  // test hook
+      wok = wok && exact_key(x) == key && exact_key(x + tot) == key;
+      if (lane == 0) {
+        if (!wok) __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        look_store(mw + kLwIncl, wok ? __double_as_longlong(x + tot) : kLookFail);
+        if (wok && b == 0) F.out[F.i0] = x;
+        S.x = x;
+        S.ok = wok ? 1 : 0;
+      }
+      unpark();
+    }
+    __syncthreads();
+    if (!S.ok) return;
+    const double xu = S.x + (incl - R);  // exact start of unit `lane`
+#pragma unroll 1
+    for (int q = 0; q < kFoldPerThread; q++, rotate(d[0]))
+      if (off0 + q * kFoldThreads < n)
+        op[fold_elem<DIR>(off0 + q * kFoldThreads)] = lane_readd(xu, 4 * q + wave) + d[0];
+    return;
+  }
+  // a block with a crossing, ties or values near zero: unit by unit
+  int k = -5000, slot = -1;
+  double R = 0.0;
+  if (ok) {
+#pragma unroll 1
+    for (int q = 0; q < kFoldPerThread; q++) {
+      const double s = wave_scan(d[0]);
+      const unsigned long long neg = __ballot(d[0] < 0.0), fin = __ballot(d[0] == d[0]);
+      const double l = (fin == ~0ULL && (neg == 0 || neg == ~0ULL)) ? fabs(s) : wave_scan(fabs(d[0]));
+      if (lane == 63) {
+        S.sum[4 * q + wave] = s;
+        S.l1[4 * q + wave] = l;
+      }
+      rotate(d[0]);
+    }
+    __syncthreads();
+    const double us = S.sum[lane], ul = S.l1[lane];
+    const double au = xs + (wave_scan(us) - us);  // approximate start of unit `lane`
+    k = sure_exponent(au, us, ul, E);
+    const int kin = sure_exponent(xs, 0.0, 0.0, E);
+    __syncthreads();
+#pragma unroll 1
+    for (int q = 0; q < kFoldPerThread; q++) {
+      const int u = 4 * q + wave, ku = __builtin_amdgcn_readlane(k, u);
+      const double du = d[0], C = ldexp(1.5, ku - 1), v = (du + C) - C;
+      double res = du;
+      if (ku > -5000) {
+        res = wave_scan(v);
+        const unsigned long long ties = __ballot(fabs(du - v) == ldexp(0.5, ku - 53));
+        if (ties) {
+          // v is the even multiple; a tie rounds to the other one when the
+          // value before it is odd, which also turns every later parity
+          const unsigned long long odd = __ballot((long long)ldexp(res - v, 53 - ku) & 1);
+          const unsigned long long up = __ballot(v < du) & ties;
+          if (lane < 2) {
+            unsigned long long flip = 0, par = lane;
+            int add = 0;
+            for (unsigned long long t = ties; t; t &= t - 1) {
+              const int i = __builtin_ctzll(t);
+              if ((par ^ (odd >> i)) & 1) {
+                flip |= 1ULL << i;
+                add += (up >> i) & 1 ? 1 : -1;
+                par ^= 1;
+              }
+            }
+            S.flip[u][lane] = flip;
+            S.adj[u][lane] = ldexp((double)add, ku - 53);
+          }
+          if (lane == 0) S.up[u] = up;
+        }
+        if (lane == 63) {
+          S.sum[u] = res;
+          S.slot[u] = ties ? -2 : -1;
+        }
+      } else {
+        // steps whose binade is open, or two binades up, leave no action to publish
+        const int ks = sure_exponent(lane_readd(au, u) + wave_scan(du), 0.0, 0.0, E);
+        const bool sure = kin > -5000 && ks > -5000 && ks <= kin + 1;
+        int row = 0;
+        if (lane == 0) {
+          row = atomicAdd(&S.nserial, 1);
+          S.slot[u] = row;
+        }
+        row = __builtin_amdgcn_readfirstlane(row);
+        if (__ballot(sure) != ~0ULL && lane == 0) S.unsure = 1;
+        if (row < kFoldSerial) S.ser[row][lane] = du;
+      }
+      rotate(res);
+    }
+    __syncthreads();
+    R = S.sum[lane];
+    slot = S.slot[lane];
+    if (slot >= 0) k = -5000;
+    ok = S.nserial <= kFoldSerial;
+  }
+  if (wave == 0) {
+    park();
+    const int kin = sure_exponent(xs, 0.0, 0.0, E);
+    bool pub = ok && b > 0 && !S.unsure && kin > -5000 && __ballot(k > kin + 1) == 0;
+    if (pub) {
+      // four consecutive starts about the approximate one, lanes 0..3 (and
+      // again in every four lanes)
+      const long long m0 = (long long)ldexp(xs, 53 - kin) & ~3LL;
+      double y = ldexp((double)(m0 + (lane & 3)), kin - 53), unused;
+      const bool good = fold_walk<false, DIR>(F, S, b, k, slot, R, y, unused);
+      const int kout = exact_key(y), kd = (kout >> 1) - (kin + 4096);
+      const bool same = kout >= 0 && kd >= -1 && kd <= 1 && (kout & 1) == (xs > 0.0 ? 1 : 0) &&
+                        kout == __builtin_amdgcn_readfirstlane(kout);
+      pub = __ballot(good && same) == ~0ULL;
+      if (pub) {
+        if (lane < 4) look_store(mw + kLwXEnd + lane, (long long)ldexp(y, 53 - ((kout >> 1) - 4096)));
+        if (lane == 0) {
+          look_store(mw + kLwXBase, m0);
+          look_store(mw + kLwXKey, ((long long)kout << 24) | ((kin + 4096) * 2 + (xs > 0.0 ? 1 : 0)));
+        }
+      }
+    }
+    if (lane == 0) look_store(mw + kLwAct, pub ? kLookCross : kLookNone);
+    double x = 0.0, xu = 0.0;
+    bool wok = ok && (b == 0 ? (x = F.x0, true) : fold_look_back(F, lw, b, S.pend, x));
+    if (W.force_replay == 2 && b == A.nblk / 2) wok = false;  // test hook
+    if (wok) {
+      if (b == 0 && lane == 0) F.out[F.i0] = x;
+      wok = fold_walk<true, DIR>(F, S, b, k, slot, R, x, xu);
+      if (!(x == x)) wok = false;  // a NaN phase takes the serial replay
+    }
+    if (lane == 0) {
+      if (!wok) __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      look_store(mw + kLwIncl, wok ? __double_as_longlong(x) : kLookFail);
+      S.ok = wok ? 1 : 0;
+    }
+    S.xu[lane] = xu;
+    unpark();
+  }
+  __syncthreads();
+  if (!S.ok) return;
+#pragma unroll 1
+  for (int q = 0; q < kFoldPerThread; q++, rotate(d[0])) {
+    const int u = 4 * q + wave;
+    const int sl = S.slot[u];
+    if (sl < 0 && off0 + q * kFoldThreads < n) {
+      double v = d[0];
+      if (sl == -2) {
+        const int ku = __builtin_amdgcn_readlane(k, u);
+        const unsigned long long f = S.flip[u][(long long)ldexp(S.xu[u], 53 - ku) & 1] & (~0ULL >> (63 - lane)), up = S.up[u];
+        v = v + ldexp((double)((int)__popcll(f & up) - (int)__popcll(f & ~up)), ku - 53);
+      }
+      op[fold_elem<DIR>(off0 + q * kFoldThreads)] = S.xu[u] + v;
     }
   }
 }
@@ -1591,8 +1810,8 @@ int fold_exact(const DenseParams &P, const DenseBuffers &B, const FoldWork &W, i
   A.nblk = (nsteps + kFoldBlock - 1) / kFoldBlock;
   if (A.nblk > nblk_cap) return -1;
   if (mode == 0) {
-    if (dir > 0) hipLaunchKernelGGL(k_fold_resolve<1>, dim3(3 * A.nblk), dim3(kFoldThreads), 0, s, A, W);
-    else hipLaunchKernelGGL(k_fold_resolve<-1>, dim3(3 * A.nblk), dim3(kFoldThreads), 0, s, A, W);
+    if (dir > 0) hipLaunchKernelGGL(k_fold_resolve<1>, dim3(A.nblk, 3), dim3(kFoldThreads), 0, s, A, W);
+    else hipLaunchKernelGGL(k_fold_resolve<-1>, dim3(A.nblk, 3), dim3(kFoldThreads), 0, s, A, W);
     // the replay check can ride on the next launch that does not read the
     // phases (the mode-sum setup); otherwise it is a launch of its own
     if (defer_replay) *defer_replay = A;
