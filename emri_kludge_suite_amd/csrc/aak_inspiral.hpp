@@ -27,6 +27,7 @@ struct Inspiral {
   double acoef[kMaxK + 2];
   double alf[kMaxK + 1][kMaxK + 1];
   double tab[4][kMaxK + 1], xtab[kMaxK + 1];
+  CircularOrbit::Hint circ;  // root of the last derivative evaluation's circular orbit
 
   AAK_HD static int nseq(int k) { return 2 * k; }
 
@@ -39,6 +40,7 @@ struct Inspiral {
     first = 1;
     kmax = kopt = 0;
     force_reset = 1;
+    circ = CircularOrbit::Hint();
     const double r_pro = Kerr::isco_pro(a), r_ret = Kerr::isco_ret(a);
     double pl, ph, pg = 0.0;
     for (int j = 1; j <= 2; j++) {
@@ -81,7 +83,7 @@ struct Inspiral {
 
   AAK_HD void derivs(const double *x, double *dx) {
     double o[3];
-    if (inspiral_rates<CX>(x[1], x[2], x[3], a, o)) {
+    if (inspiral_rates<CX>(x[1], x[2], x[3], a, o, &circ)) {
       err = 1;
       o[0] = o[1] = o[2] = NAN;
     }
