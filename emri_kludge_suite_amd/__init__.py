@@ -2,7 +2,7 @@
 Suite's GPU path: pygpuAAK's GPUAAK class and the gpuAAK.h entry points).
 
 The compute runs in the in-tree HIP library libaak_hip.so (hand-written
-gfx950 kernels + rocFFT) behind the C ABI declared in include/gpuAAK.h.
+gfx950 kernels; rocFFT for some lengths) behind the C ABI declared in include/gpuAAK.h.
 
   GPUAAK       the reference's GPUAAK class (plus LikelihoodBatch)
   OmegaPhi, PNevolution   the free functions of the reference's gpuAAK.h

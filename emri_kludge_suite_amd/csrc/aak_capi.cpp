@@ -10,8 +10,10 @@
 //     one template's narrow kernels overlap another's wide ones,
 //   * the inner-product stage: for power-of-two lengths the fused four-step
 //     FFT + weighted reduction (aak_fft.hip, data stored in its row order),
-//     otherwise a rocFFT real-forward plan per lane (both channels in one
-//     batched call) and the separate reduction; the Bessel tables,
+//     for lengths whose half has a prime factor above 13 the convolution of
+//     the same file, otherwise a rocFFT real-forward plan per lane (both
+//     channels in one batched call) and the separate reduction; the Bessel
+//     tables,
 //   * for batches, a pool of host threads and a ring of plan slots whose knot
 //     tables live in pinned host memory.
 //
@@ -196,7 +198,8 @@ struct Lane {
   int fold_nblk_cap = 0;
   void *d_foldmem = nullptr;
   double2 *d_hf = nullptr;    // [2][nbins]
-  double2 *d_fy = nullptr;    // [2][N/2] four-step FFT scratch (fused FFT path)
+  double2 *d_fy = nullptr;    // [2][N/2] four-step FFT scratch (fused FFT path); [2][L] (chirp)
+  double2 *d_fz = nullptr;    // [2][N/2] transforms before the real-spectrum split (chirp)
   double *d_partials = nullptr, *d_like = nullptr;
   double *d_fparts = nullptr;     // pass 2 with the final reduction: published pairs
   double *d_ms_coef = nullptr;  // mode-sum block Taylor coefficients (grown with nmodes)
@@ -234,8 +237,10 @@ struct aak_handle_s {
   double *d_bessel = nullptr;     // c_m(k) table | log k!
   double2 *d_data = nullptr;      // [2][nbins] weighted data (fused FFT path: in its row order)
   double *d_w = nullptr;          // [2][nbins] weights (same order as d_data)
-  bool fused_fft = false;         // power-of-two length: fused FFT + reduction, else rocFFT
+  bool fused_fft = false;         // power-of-two length: fused FFT + reduction
+  bool chirp_fft = false;         // N/2 with a prime factor above 13: Bluestein's convolution, else rocFFT
   FftArgs fft{};
+  ChirpArgs chirp{};
   double2 *d_fft_tw = nullptr;    // twiddle tables of the fused FFT
   double *d_like_batch = nullptr;
   double *d_phase = nullptr;      // [8][N] phase output, allocated on first use
@@ -376,7 +381,7 @@ static int alloc_lane(aak_handle h, Lane &L) {
   L.fold_reset = FoldReset{L.fw.look, (int)(2 * 3 * (size_t)nblk * kLW), L.fw.status, L.fw.look_ctr, 0};
   const int nb = h->nbins;
   HIPCHK(hipMalloc(&L.d_hf, sizeof(double2) * 2 * (size_t)nb));
-  const int nparts = std::max(2048, h->fused_fft ? fft_partials(h->fft) : 0);
+  const int nparts = std::max(2048, h->fused_fft ? fft_partials(h->fft) : h->chirp_fft ? chirp_partials(h->chirp) : 0);
   HIPCHK(hipMalloc(&L.d_partials, sizeof(double) * 2 * (size_t)nparts));
   HIPCHK(hipMalloc(&L.d_like, sizeof(double) * 2));
   if (h->fused_fft) {
@@ -385,6 +390,12 @@ static int alloc_lane(aak_handle h, Lane &L) {
     HIPCHK(hipMalloc(&L.d_fparts, sizeof(double) * 2 * (size_t)fp));
     launch_fft_final_reset(L.d_fparts, fp, L.stream);
     HIPCHK(hipGetLastError());
+    L.ready = true;
+    return 0;
+  }
+  if (h->chirp_fft) {
+    HIPCHK(hipMalloc(&L.d_fy, sizeof(double2) * 2 * (size_t)h->chirp.L));
+    HIPCHK(hipMalloc(&L.d_fz, sizeof(double2) * 2 * (size_t)h->chirp.M));
     L.ready = true;
     return 0;
   }
@@ -424,7 +435,7 @@ static void free_lane(Lane &L) {
   if (L.plan) rocfft_plan_destroy(L.plan);
   if (L.exec) rocfft_execution_info_destroy(L.exec);
   void *ptrs[] = {L.d_table[0], L.d_table[1], L.d_dense, L.d_h, L.d_t, L.d_flags, L.d_guardw, L.d_foldmem,
-                  L.d_hf, L.d_fy, L.d_partials, L.d_fparts, L.d_like, L.d_work, L.d_ms_coef, L.d_ms_p, L.d_ms_slot,
+                  L.d_hf, L.d_fy, L.d_fz, L.d_partials, L.d_fparts, L.d_like, L.d_work, L.d_ms_coef, L.d_ms_p, L.d_ms_slot,
                   L.d_ms_list, L.d_ms_split, L.d_ms_eref};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -460,6 +471,21 @@ static int alloc_handle(aak_handle h) {
     F.Dp[1] = h->d_data + nb;
     F.wp[0] = h->d_w;
     F.wp[1] = h->d_w + nb;
+  }
+  int rc = 0;
+  if (h->chirp_fft) {
+    ChirpArgs &F = h->chirp;
+    std::vector<double2> tw(chirp_host_tables(F, nullptr));
+    chirp_host_tables(F, tw.data());
+    HIPCHK(hipMalloc(&h->d_fft_tw, sizeof(double2) * chirp_table_size(F)));
+    HIPCHK(hipMemcpy(h->d_fft_tw, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice));
+    chirp_bind_tables(&F, h->d_fft_tw);
+    if ((rc = alloc_lane(h, h->lane[0]))) return rc;
+    // on lane 0's stream, waited for here: other lanes read the tables too
+    launch_chirp_init(F, h->d_fft_tw, h->lane[0].d_fy, h->lane[0].stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(h->lane[0].stream));
+    return 0;
   }
   return alloc_lane(h, h->lane[0]);
 }
@@ -629,6 +655,16 @@ static int enqueue_likelihood(aak_handle h, Lane &L, double *out_dev, bool keep_
     h->mark(L, 4);
     launch_fft_pass2(h->fft, L.d_fy, L.d_partials, keep_spectrum ? L.d_hf : nullptr, L.stream);
     launch_dot_final(L.d_partials, fft_partials(h->fft), out_dev, flags, clear, L.stream);
+    h->mark(L, 5);
+    HIPCHK(hipGetLastError());
+    if (clear) L.flags_dirty = false;
+    return 0;
+  }
+  if (h->chirp_fft) {
+    launch_chirp_fft(h->chirp, L.d_h, L.d_h + h_stride(h->N), L.d_fy, L.d_fz, L.stream);
+    h->mark(L, 4);
+    launch_chirp_dot(h->chirp, L.d_fz, h->d_data, h->d_w, keep_spectrum ? L.d_hf : nullptr, L.d_partials, L.stream);
+    launch_dot_final(L.d_partials, chirp_partials(h->chirp), out_dev, flags, clear, L.stream);
     h->mark(L, 5);
     HIPCHK(hipGetLastError());
     if (clear) L.flags_dirty = false;
@@ -867,13 +903,21 @@ int aak_create(double T_fit, int init_length, int length, double init_dt, double
   {
     // AAK_FFT=rocfft keeps the library transform for every length
     const char *env = std::getenv("AAK_FFT");
+    const bool library = env && std::strcmp(env, "rocfft") == 0;
     int R = 0, C = 0;
-    if (!(env && std::strcmp(env, "rocfft") == 0) && fft_supported(length, &R, &C)) {
+    if (!library && fft_supported(length, &R, &C)) {
       h->fused_fft = true;
       h->fft.N = length;
       h->fft.M = length / 2;
       h->fft.R = R;
       h->fft.C = C;
+    } else if (!library && chirp_supported(length, &R, &C)) {
+      h->chirp_fft = true;
+      h->chirp.N = length;
+      h->chirp.M = length / 2;
+      h->chirp.L = R * C;
+      h->chirp.R = R;
+      h->chirp.C = C;
     }
   }
   const int rc = alloc_handle(h);

@@ -38,8 +38,12 @@ __device__ inline double2 cmul_mi(double2 a) { return make_double2(a.y, -a.x); }
 constexpr double kC8 = 0.92387953251128675613;
 constexpr double kS8 = 0.38268343236508977173;
 constexpr double kR2 = 0.70710678118654752440;
+constexpr double kS3 = 0.86602540378443864676;  // sin(2 pi / 3)
+constexpr double kC20 = 0.93969262078590838405, kS20 = 0.34202014332566873304;  // cos, sin of 20 degrees,
+constexpr double kC40 = 0.76604444311897803520, kS40 = 0.64278760968653932632;  // 40 and
+constexpr double kC80 = 0.17364817766693034885, kS80 = 0.98480775301220805937;  // 80
 
-__device__ inline void dft4(double2 &a0, double2 &a1, double2 &a2, double2 &a3) {
+__device__ __forceinline__ void dft4(double2 &a0, double2 &a1, double2 &a2, double2 &a3) {
   const double2 t0 = cadd(a0, a2), t1 = csub(a0, a2), t2 = cadd(a1, a3), t3 = cmul_mi(csub(a1, a3));
   a0 = cadd(t0, t2);
   a1 = cadd(t1, t3);
@@ -47,12 +51,52 @@ __device__ inline void dft4(double2 &a0, double2 &a1, double2 &a2, double2 &a3) 
   a3 = csub(t1, t3);
 }
 
+__device__ __forceinline__ void dft3(double2 &a0, double2 &a1, double2 &a2) {
+  const double2 t = cadd(a1, a2), u = cmul_mi(csub(a1, a2));
+  const double2 c = make_double2(a0.x - 0.5 * t.x, a0.y - 0.5 * t.y);
+  a0 = cadd(a0, t);
+  a1 = make_double2(c.x + kS3 * u.x, c.y + kS3 * u.y);
+  a2 = make_double2(c.x - kS3 * u.x, c.y - kS3 * u.y);
+}
+
 // Forward DFT of RS points, v in natural order, o out in natural order.
 template <int RS>
-__device__ inline void dft(double2 *v, double2 *o) {
+__device__ __forceinline__ void dft(double2 *v, double2 *o) {
   if constexpr (RS == 2) {
     o[0] = cadd(v[0], v[1]);
     o[1] = csub(v[0], v[1]);
+  } else if constexpr (RS == 9) {
+    // n = 3 n1 + n2, k = k1 + 3 k2
+#pragma unroll
+    for (int n2 = 0; n2 < 3; n2++) dft3(v[n2], v[3 + n2], v[6 + n2]);
+    // v[n2 + 3 k1] *= W9^(n2 k1)
+    v[4] = cmul(v[4], make_double2(kC40, -kS40));
+    v[5] = cmul(v[5], make_double2(kC80, -kS80));
+    v[7] = cmul(v[7], make_double2(kC80, -kS80));
+    v[8] = cmul(v[8], make_double2(-kC20, -kS20));
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++) dft3(v[3 * k1], v[3 * k1 + 1], v[3 * k1 + 2]);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++)
+#pragma unroll
+      for (int k2 = 0; k2 < 3; k2++) o[k1 + 3 * k2] = v[3 * k1 + k2];
+  } else if constexpr (RS == 12) {
+    // n = 4 n1 + n2, k = k1 + 3 k2
+#pragma unroll
+    for (int n2 = 0; n2 < 4; n2++) dft3(v[n2], v[4 + n2], v[8 + n2]);
+    // v[n2 + 4 k1] *= W12^(n2 k1)
+    v[5] = cmul(v[5], make_double2(kS3, -0.5));
+    v[6] = cmul(v[6], make_double2(0.5, -kS3));
+    v[7] = cmul_mi(v[7]);
+    v[9] = cmul(v[9], make_double2(0.5, -kS3));
+    v[10] = cmul(v[10], make_double2(-0.5, -kS3));
+    v[11] = make_double2(-v[11].x, -v[11].y);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++) dft4(v[4 * k1], v[4 * k1 + 1], v[4 * k1 + 2], v[4 * k1 + 3]);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; k1++)
+#pragma unroll
+      for (int k2 = 0; k2 < 4; k2++) o[k1 + 3 * k2] = v[4 * k1 + k2];
   } else if constexpr (RS == 4) {
     dft4(v[0], v[1], v[2], v[3]);
 #pragma unroll
@@ -70,7 +114,7 @@ __device__ inline void dft(double2 *v, double2 *o) {
       o[k1 + 4] = csub(v[2 * k1], v[2 * k1 + 1]);
     }
   } else {
-    static_assert(RS == 16, "radix 2, 4, 8 or 16");
+    static_assert(RS == 16, "radix 2, 4, 8, 9, 12 or 16");
     // n = 4 n1 + n2, k = k1 + 4 k2
 #pragma unroll
     for (int n2 = 0; n2 < 4; n2++) dft4(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
@@ -94,17 +138,24 @@ __device__ inline void dft(double2 *v, double2 *o) {
 }
 
 constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x / 2); }
-// radix of the stage that faces `rem` remaining points: 16 while that leaves a
-// power of 16 or at least 4 behind, then 8, 4 or 2
+// radix of the stage that faces `rem` remaining points: a factor of 9 or 3 first,
+// then 16 while that leaves a power of 16 or at least 4 behind, then 8, 4 or 2
 constexpr int stage_radix(int rem) {
-  return (ilog2(rem) >= 4 && ilog2(rem) != 5) ? 16 : (ilog2(rem) == 5 ? 8 : rem);
+  return rem % 9 == 0                               ? 9
+         : rem % 3 == 0                             ? 12
+         : (ilog2(rem) >= 4 && ilog2(rem) != 5)     ? 16
+         : ilog2(rem) == 5                          ? 8
+                                                    : rem;
 }
 
 __device__ inline int pad(int i) { return i + (i >> 4); }
 
+// The stages are forced inline: shared by many kernels they would become calls,
+// which cost the two passes 5 us of 66 per inner product at N = 2^21.
 // One Stockham stage of radix RS on L points held in x (LDS, padded), NT threads.
-template <int L, int NT, int NS, int RS>
-__device__ inline void fft_stage(double2 *x, int t, const double2 *tw) {
+// MUL (first stage only): the points are read as conj(x f), f in global memory.
+template <int L, int NT, int NS, int RS, bool MUL = false>
+__device__ __forceinline__ void fft_stage(double2 *x, int t, const double2 *tw, const double2 *f = nullptr) {
   constexpr int NB = L / RS;
   constexpr int PER = (NB + NT - 1) / NT;
   double2 o[PER][RS];
@@ -112,13 +163,20 @@ __device__ inline void fft_stage(double2 *x, int t, const double2 *tw) {
   for (int u = 0; u < PER; u++) {
     const int j = t + u * NT;
     if (NB % NT == 0 || j < NB) {
-      const int jm = j & (NS - 1);
+      const int jm = (unsigned)j % NS;
       double2 v[RS];
 #pragma unroll
       for (int r = 0; r < RS; r++) v[r] = x[pad(j + r * NB)];
+      if constexpr (MUL) {
+#pragma unroll
+        for (int r = 0; r < RS; r++) {
+          const double2 m = cmul(v[r], f[j + r * NB]);
+          v[r] = make_double2(m.x, -m.y);
+        }
+      }
       if constexpr (NS > 1) {
 #pragma unroll
-        for (int r = 1; r < RS; r++) v[r] = cmul(v[r], tw[(r * jm * (L / (RS * NS))) & (L - 1)]);
+        for (int r = 1; r < RS; r++) v[r] = cmul(v[r], tw[r * jm * (L / (RS * NS))]);
       }
       dft<RS>(v, o[u]);
     }
@@ -128,7 +186,7 @@ __device__ inline void fft_stage(double2 *x, int t, const double2 *tw) {
   for (int u = 0; u < PER; u++) {
     const int j = t + u * NT;
     if (NB % NT == 0 || j < NB) {
-      const int d = (j / NS) * NS * RS + (j & (NS - 1));
+      const int d = (unsigned)j / NS * NS * RS + (unsigned)j % NS;
 #pragma unroll
       for (int r = 0; r < RS; r++) x[pad(d + r * NS)] = o[u][r];
     }
@@ -137,7 +195,7 @@ __device__ inline void fft_stage(double2 *x, int t, const double2 *tw) {
 }
 
 template <int L, int NT, int NS>
-__device__ inline void fft_stages(double2 *x, int t, const double2 *tw) {
+__device__ __forceinline__ void fft_stages(double2 *x, int t, const double2 *tw) {
   if constexpr (NS < L) {
     constexpr int RS = stage_radix(L / NS);
     fft_stage<L, NT, NS, RS>(x, t, tw);
@@ -145,11 +203,19 @@ __device__ inline void fft_stages(double2 *x, int t, const double2 *tw) {
   }
 }
 
+// Whole L-point FFT of conj(x f).
+template <int L, int NT>
+__device__ __forceinline__ void fft_conj_product(double2 *x, int t, const double2 *tw, const double2 *f) {
+  constexpr int RS = stage_radix(L);
+  fft_stage<L, NT, 1, RS, true>(x, t, tw, f);
+  fft_stages<L, NT, RS>(x, t, tw);
+}
+
 // Whole L-point FFT whose first stage (no twiddles) reads straight from global
 // memory: butterfly j reads src[j + r L / RS], contiguous across the threads
 // for each r.
 template <int L, int NT>
-__device__ inline void fft_first_global(const double2 *src, double2 *x, int t, const double2 *tw) {
+__device__ __forceinline__ void fft_first_global(const double2 *src, double2 *x, int t, const double2 *tw) {
   constexpr int RS = stage_radix(L);
   constexpr int NB = L / RS;
   constexpr int PER = (NB + NT - 1) / NT;
@@ -183,20 +249,20 @@ constexpr int col_cols() { return LR <= 512 ? 8 : 4; }
 // start on different banks
 template <int LR>
 constexpr int col_stride() { return LR + LR / 16 + 1; }
-// threads per column or row: one radix-16 butterfly each in the first stage
+// threads per column or row: one butterfly each in the first stage (16, 12 or 9
+// points), in whole waves
 template <int L>
-constexpr int fft_threads() { return L / 16 > 64 ? L / 16 : 64; }
+constexpr int fft_threads() { return L <= 1024 ? 64 : L % 3 == 0 ? L / stage_radix(L) : L / 16; }
 
-template <int LR>
-__global__ __launch_bounds__(col_cols<LR>() * fft_threads<LR>()) void k_fft_cols(FftArgs F, const double *h0,
-                                                                                  const double *h1, double2 *Y) {
-  constexpr int CC = col_cols<LR>(), CS = col_stride<LR>(), NT = fft_threads<LR>();
-  __shared__ double2 s[CC * CS];
-  int ch = blockIdx.y, grp = blockIdx.x;
+// Channel and column group of a workgroup.  Workgroups are dealt round-robin to
+// the 8 XCDs in launch order; groups 2q and 2q + 1 of half a 128-byte line
+// per row are paired on one XCD, launched 8 apart, so each line is fetched
+// into one L2 once.
+template <int CC>
+__device__ inline void col_group(int &ch, int &grp) {
+  ch = blockIdx.y;
+  grp = blockIdx.x;
   if (CC < 8) {
-    // workgroups are dealt round-robin to the 8 XCDs in launch order; pair
-    // groups 2q and 2q+1 (one 128-byte line per row between them) on one XCD,
-    // launched 8 apart, so each line is fetched into one L2 once
     const int L = blockIdx.y * gridDim.x + blockIdx.x, total = gridDim.x * gridDim.y;
     if ((total & 15) == 0) {
       const int xcd = L & 7, r = L >> 3;
@@ -205,6 +271,15 @@ __global__ __launch_bounds__(col_cols<LR>() * fft_threads<LR>()) void k_fft_cols
       grp = g % gridDim.x;
     }
   }
+}
+
+template <int LR>
+__global__ __launch_bounds__(col_cols<LR>() * fft_threads<LR>()) void k_fft_cols(FftArgs F, const double *h0,
+                                                                                  const double *h1, double2 *Y) {
+  constexpr int CC = col_cols<LR>(), CS = col_stride<LR>(), NT = fft_threads<LR>();
+  __shared__ double2 s[CC * CS];
+  int ch, grp;
+  col_group<CC>(ch, grp);
   const int b0 = grp * CC, tid = threadIdx.x;
   constexpr int PT = (LR + NT - 1) / NT;  // elements per thread in the staging loops
   constexpr bool kFull = LR % NT == 0;
@@ -437,6 +512,200 @@ __global__ __launch_bounds__(2 * fft_threads<LC>()) void k_fft_rows(FftArgs F, c
   }
 }
 
+// ---------------------------------------------------------------- other lengths
+// The M-point transform of a length N = 2M that the passes above do not take,
+// as Bluestein's convolution (L. Bluestein, 1970): with c_m = exp(-i pi m^2 / M),
+//   Z_k = c_k sum_m (z_m c_m) conj(c_(k-m)),
+// a cyclic convolution of length L >= 2M - 1 with a fixed filter, whose
+// transform F is formed once per handle.  L = R C with R from 2^a, C from 2^a,
+// 3 2^a and 9 2^a, at most a third longer than it must be from N = 512 on.
+// Both transforms of the convolution run in the four-step form above, and what
+// lies between them stays in LDS:
+//   k_chirp_cols   columns b of z_m c_m (zero from M on), times W_L^(b k1);
+//   k_chirp_rows   rows k1: forward FFT, times F, inverse FFT, times
+//                  W_L^(-b k1), in place;
+//   k_chirp_back   columns b back to m = a C + b < M, times c_m;
+//   k_chirp_dot    the real spectrum from Z_k and Z_(M-k), weighting, both sums.
+// Inverse transforms are conjugated forward ones; F carries their 1/L.
+// At N = 2103840 (1024 x 2304) the four kernels move 0.48 GB and take 53 + 69 +
+// 40 + 14 us, 196 us per likelihood with the final sum, where the library's
+// transform took 781 us in twelve kernels.  Factors 9 and 12 as one stage each
+// and one row per workgroup (four of 256 threads per CU share the LDS) matter
+// most to the rows: 111 us with radices 16, 16, 3, 3 and two rows per workgroup.
+// A 1536 x 1536 split took 84 + 91 + 76 us: 104 KB of LDS for 4 columns leaves
+// one workgroup per CU.  Against 80-bit transforms the spectrum's error is
+// 6e-16 (relative L2), the library's 1.1e-15.
+__device__ inline double2 conjd(double2 a) { return make_double2(a.x, -a.y); }
+
+__global__ void k_chirp_table(double2 *c, int M) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= M) return;
+  // m^2 mod 2M in integers: the angle is exact before its one rounding
+  const long long q = ((long long)m * m) % (2LL * M);
+  double sn, cs;
+  sincospi((double)q / (double)M, &sn, &cs);
+  c[m] = make_double2(cs, -sn);
+}
+
+// FILTER: the columns of the filter conj(c_|m|) instead of a channel.
+template <int LR, bool FILTER>
+__global__ __launch_bounds__(col_cols<LR>() * fft_threads<LR>()) void k_chirp_cols(ChirpArgs F, const double *h0,
+                                                                                   const double *h1, double2 *Y) {
+  constexpr int CC = col_cols<LR>(), CS = col_stride<LR>(), NT = fft_threads<LR>();
+  __shared__ double2 s[CC * CS];
+  int ch, grp;
+  col_group<CC>(ch, grp);
+  const int b0 = grp * CC, tid = threadIdx.x;
+  constexpr int PT = (LR + NT - 1) / NT;
+  const double2 *z = reinterpret_cast<const double2 *>(ch ? h1 : h0);
+  {
+    double2 v[PT], c[PT];
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+      const int idx = tid + q * CC * NT;
+      const int m = (idx / CC) * F.C + b0 + idx % CC;
+      v[q] = c[q] = make_double2(0.0, 0.0);
+      if (idx < CC * LR) {
+        if (FILTER) {
+          const int j = m < F.M ? m : F.L - m;
+          if (j < F.M) c[q] = F.chirp[j];
+        } else if (m < F.M) {
+          v[q] = z[m];
+          c[q] = F.chirp[m];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+      const int idx = tid + q * CC * NT;
+      if (idx < CC * LR) s[(idx % CC) * CS + pad(idx / CC)] = FILTER ? conjd(c[q]) : cmul(v[q], c[q]);
+    }
+  }
+  __syncthreads();
+  fft_stages<LR, NT, 1>(s + (tid / NT) * CS, tid % NT, F.twR);
+  double2 *Yc = Y + (size_t)ch * F.L;
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const int idx = tid + q * CC * NT;
+    const int k1 = idx / CC, c = idx % CC, b = b0 + c;
+    if (idx < CC * LR)
+      Yc[(size_t)k1 * F.C + b] = cmul(s[c * CS + pad(k1)], tw2(F.twLhi, F.twLlo, (long long)b * k1));
+  }
+}
+
+// One row per workgroup.  FILTER: the filter's transform (with the 1/L) goes to
+// Fo in the order of the rows.
+template <int LC, bool FILTER>
+__global__ __launch_bounds__(fft_threads<LC>()) void k_chirp_rows(ChirpArgs F, double2 *Y, double2 *Fo) {
+  constexpr int NT = fft_threads<LC>(), PT = (LC + NT - 1) / NT;
+  __shared__ double2 x[LC + LC / 16];
+  const int ch = blockIdx.y, t = threadIdx.x, k1 = blockIdx.x;
+  double2 *row = Y + (size_t)ch * F.L + (size_t)k1 * F.C;
+  fft_first_global<LC, NT>(row, x, t, F.twC);
+  const size_t f0 = (size_t)k1 * F.C;
+  if (FILTER) {
+    const double inv = 1.0 / (double)F.L;
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+      const int k2 = t + q * NT;
+      if (k2 < LC) Fo[f0 + k2] = make_double2(x[pad(k2)].x * inv, x[pad(k2)].y * inv);
+    }
+    return;
+  }
+  fft_conj_product<LC, NT>(x, t, F.twC, F.filter + f0);
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const int b = t + q * NT;
+    if (b < LC) row[b] = conjd(cmul(x[pad(b)], tw2(F.twLhi, F.twLlo, (long long)b * k1)));
+  }
+}
+
+template <int LR>
+__global__ __launch_bounds__(col_cols<LR>() * fft_threads<LR>()) void k_chirp_back(ChirpArgs F, const double2 *Y,
+                                                                                   double2 *Z) {
+  constexpr int CC = col_cols<LR>(), CS = col_stride<LR>(), NT = fft_threads<LR>();
+  __shared__ double2 s[CC * CS];
+  int ch, grp;
+  col_group<CC>(ch, grp);
+  const int b0 = grp * CC, tid = threadIdx.x;
+  constexpr int PT = (LR + NT - 1) / NT;
+  const double2 *Yc = Y + (size_t)ch * F.L;
+  double2 *Zc = Z + (size_t)ch * F.M;
+  {
+    double2 v[PT];
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+      const int idx = tid + q * CC * NT;
+      v[q] = make_double2(0.0, 0.0);
+      if (idx < CC * LR) v[q] = Yc[(size_t)(idx / CC) * F.C + b0 + idx % CC];
+    }
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+      const int idx = tid + q * CC * NT;
+      if (idx < CC * LR) s[(idx % CC) * CS + pad(idx / CC)] = conjd(v[q]);
+    }
+  }
+  __syncthreads();
+  fft_stages<LR, NT, 1>(s + (tid / NT) * CS, tid % NT, F.twR);
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const int idx = tid + q * CC * NT;
+    const int m = (idx / CC) * F.C + b0 + idx % CC;
+    if (idx < CC * LR && m < F.M) Zc[m] = cmul(conjd(s[(idx % CC) * CS + pad(idx / CC)]), F.chirp[m]);
+  }
+}
+
+// H_k and H_(M-k) of one pair (k <= M/2) from Z_k and Z_(M-k), weighted and
+// summed over both channels.
+constexpr int kPairThreads = 256, kPairBlocks = 1024;
+__global__ __launch_bounds__(kPairThreads) void k_chirp_dot(ChirpArgs F, const double2 *Z, const double2 *data,
+                                                            const double *w, double2 *hw_out, double *partials) {
+  __shared__ double s_red[kPairThreads / 64][2];
+  const int M = F.M, nb = M + 1, half = M / 2 + 1, tid = threadIdx.x;
+  double dh = 0.0, hh = 0.0;
+  for (int q = blockIdx.x * kPairThreads + tid; q < 2 * half; q += gridDim.x * kPairThreads) {
+    const int ch = q >= half, k = q - ch * half, j = M - k;
+    const double2 *Zc = Z + (size_t)ch * M;
+    const double2 *dc = data + (size_t)ch * nb;
+    const double *wc = w + (size_t)ch * nb;
+    double2 *hc = hw_out ? hw_out + (size_t)ch * nb : nullptr;
+    const double2 zk = Zc[k], zm = k == 0 ? zk : Zc[j];
+    const double2 dk = dc[k], dj = dc[j];
+    const double wk = wc[k], wj = wc[j];
+    const double2 E = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+    const double2 O = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+    const double2 WO = cmul(tw2(F.twNhi, F.twNlo, k), O);
+    // H_k = E + W O, H_(M-k) = conj(E - W O)
+    const double2 a = make_double2((E.x + WO.x) * wk, (E.y + WO.y) * wk);
+    const double2 b = make_double2((E.x - WO.x) * wj, -(E.y - WO.y) * wj);
+    dh += a.x * dk.x + a.y * dk.y;
+    hh += a.x * a.x + a.y * a.y;
+    if (hc) hc[k] = a;
+    if (j != k) {
+      dh += b.x * dj.x + b.y * dj.y;
+      hh += b.x * b.x + b.y * b.y;
+      if (hc) hc[j] = b;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    dh += __shfl_xor(dh, o, 64);
+    hh += __shfl_xor(hh, o, 64);
+  }
+  if ((tid & 63) == 0) {
+    s_red[tid >> 6][0] = dh;
+    s_red[tid >> 6][1] = hh;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int v = 1; v < kPairThreads / 64; v++) {
+      dh += s_red[v][0];
+      hh += s_red[v][1];
+    }
+    partials[2 * blockIdx.x] = dh;
+    partials[2 * blockIdx.x + 1] = hh;
+  }
+}
+
 // ---------------------------------------------------------------- launch
 template <int LR>
 static void launch_cols(const FftArgs &F, const double *h0, const double *h1, double2 *Y, hipStream_t s) {
@@ -559,6 +828,183 @@ void launch_fft_pass2_final(const FftArgs &F, const double2 *Y, double *partials
 
 void launch_fft_final_reset(double *partials, int npairs, hipStream_t s) {
   hipLaunchKernelGGL(k_fft_final_reset, dim3(8), dim3(256), 0, s, partials, 2 * npairs);
+}
+
+// ---------------------------------------------------------------- other lengths
+// Columns of 2^a points, rows of 2^a, 3 2^a or 9 2^a.
+static const int kChirpRows[] = {16,  32,  48,  64,  96,  128, 144,  192,  256, 288,
+                                 384, 512, 576, 768, 1024, 1152, 1536, 2048, 2304};
+
+// Lengths whose half is a product of primes up to 13 stay with the library's
+// mixed-radix transforms, which need no convolution for them: at N = 2000000 they
+// take 106 us against 183 of the convolution, at 250000 39 against 46, at 4000
+// 22 against 29.  For all others the library runs a convolution too, and this
+// one is faster throughout (N = 2103840: 196 us against 781, 1048578: 107
+// against 384, 65538: 37 against 56, 4002: 29 against 44, 1002: 23 against 30).
+bool chirp_supported(int N, int *R, int *C) {
+  if (N < 16 || (N & 1)) return false;
+  int rest = N / 2;
+  for (int q : {2, 3, 5, 7, 11, 13})
+    while (rest % q == 0) rest /= q;
+  if (rest == 1) return false;
+  const long long need = (long long)N - 1;  // 2M - 1
+  long long best = 0;
+  for (int r = 16; r <= 2048; r *= 2)
+    for (int c : kChirpRows) {
+      // the shortest product; columns no longer than rows leave two workgroups
+      // per CU (1024-point columns); only 2048 x 1536 has no such form
+      const long long l = (long long)r * c;
+      if (l < need || (c < r && c != 1536)) continue;
+      if (best == 0 || l < best || (l == best && r > *R)) {
+        best = l;
+        *R = r;
+        *C = c;
+      }
+    }
+  return best != 0;
+}
+
+int chirp_partials(const ChirpArgs &F) {
+  const int need = (2 * (F.M / 2 + 1) + kPairThreads - 1) / kPairThreads;
+  return need < kPairBlocks ? need : kPairBlocks;
+}
+
+// Table layout: W_R | W_C | W_L lo | W_L hi | W_N lo | W_N hi, then the chirp
+// and the filter's transform, which the device forms.
+static void chirp_offsets(const ChirpArgs &F, size_t o[9]) {
+  o[0] = 0;
+  o[1] = o[0] + F.R;
+  o[2] = o[1] + F.C;
+  o[3] = o[2] + 1024;
+  o[4] = o[3] + (size_t)F.L / 1024 + 2;
+  o[5] = o[4] + 1024;
+  o[6] = o[5] + (size_t)F.M / 1024 + 2;
+  o[7] = o[6] + F.M;
+  o[8] = o[7] + F.L;
+}
+
+size_t chirp_table_size(const ChirpArgs &F) {
+  size_t o[9];
+  chirp_offsets(F, o);
+  return o[8];
+}
+
+size_t chirp_host_tables(const ChirpArgs &F, double2 *tw) {
+  size_t o[9];
+  chirp_offsets(F, o);
+  if (!tw) return o[6];
+  auto root = [](long long e, long long L) {
+    const long double pi = 3.141592653589793238462643383279502884L;
+    const long double a = -2.0L * pi * (long double)(e % L) / (long double)L;
+    return make_double2((double)cosl(a), (double)sinl(a));
+  };
+  for (int e = 0; e < F.R; e++) tw[o[0] + e] = root(e, F.R);
+  for (int e = 0; e < F.C; e++) tw[o[1] + e] = root(e, F.C);
+  for (int e = 0; e < 1024; e++) {
+    tw[o[2] + e] = root(e, F.L);
+    tw[o[4] + e] = root(e, F.N);
+  }
+  for (size_t e = 0; e < o[4] - o[3]; e++) tw[o[3] + e] = root(1024LL * e, F.L);
+  for (size_t e = 0; e < o[6] - o[5]; e++) tw[o[5] + e] = root(1024LL * e, F.N);
+  return o[6];
+}
+
+void chirp_bind_tables(ChirpArgs *F, double2 *tw) {
+  size_t o[9];
+  chirp_offsets(*F, o);
+  F->twR = tw + o[0];
+  F->twC = tw + o[1];
+  F->twLlo = tw + o[2];
+  F->twLhi = tw + o[3];
+  F->twNlo = tw + o[4];
+  F->twNhi = tw + o[5];
+  F->chirp = tw + o[6];
+  F->filter = tw + o[7];
+}
+
+namespace {
+struct ChirpCall {
+  const ChirpArgs &F;
+  const double *h0, *h1;
+  double2 *Y, *Z, *Fo;
+  hipStream_t s;
+};
+template <int S>
+void chirp_cols(const ChirpCall &c, bool filter) {
+  const dim3 grid(c.F.C / col_cols<S>(), filter ? 1 : 2), block(col_cols<S>() * fft_threads<S>());
+  if (filter) hipLaunchKernelGGL((k_chirp_cols<S, true>), grid, block, 0, c.s, c.F, nullptr, nullptr, c.Y);
+  else hipLaunchKernelGGL((k_chirp_cols<S, false>), grid, block, 0, c.s, c.F, c.h0, c.h1, c.Y);
+}
+template <int S>
+void chirp_rows(const ChirpCall &c, bool filter) {
+  const dim3 grid(c.F.R, filter ? 1 : 2), block(fft_threads<S>());
+  if (filter) hipLaunchKernelGGL((k_chirp_rows<S, true>), grid, block, 0, c.s, c.F, c.Y, c.Fo);
+  else hipLaunchKernelGGL((k_chirp_rows<S, false>), grid, block, 0, c.s, c.F, c.Y, nullptr);
+}
+template <int S>
+void chirp_back(const ChirpCall &c) {
+  hipLaunchKernelGGL(k_chirp_back<S>, dim3(c.F.C / col_cols<S>(), 2), dim3(col_cols<S>() * fft_threads<S>()), 0, c.s,
+                     c.F, c.Y, c.Z);
+}
+#define CHIRP_POW2(fn, ...)                     \
+    case 16: fn<16>(__VA_ARGS__); break;        \
+    case 32: fn<32>(__VA_ARGS__); break;        \
+    case 64: fn<64>(__VA_ARGS__); break;        \
+    case 128: fn<128>(__VA_ARGS__); break;      \
+    case 256: fn<256>(__VA_ARGS__); break;      \
+    case 512: fn<512>(__VA_ARGS__); break;      \
+    case 1024: fn<1024>(__VA_ARGS__); break;
+void chirp_cols_of(const ChirpCall &c, bool filter) {
+  switch (c.F.R) {
+    CHIRP_POW2(chirp_cols, c, filter)
+    default: chirp_cols<2048>(c, filter); break;
+  }
+}
+void chirp_back_of(const ChirpCall &c) {
+  switch (c.F.R) {
+    CHIRP_POW2(chirp_back, c)
+    default: chirp_back<2048>(c); break;
+  }
+}
+void chirp_rows_of(const ChirpCall &c, bool filter) {
+  switch (c.F.C) {
+    CHIRP_POW2(chirp_rows, c, filter)
+    case 48: chirp_rows<48>(c, filter); break;
+    case 96: chirp_rows<96>(c, filter); break;
+    case 144: chirp_rows<144>(c, filter); break;
+    case 192: chirp_rows<192>(c, filter); break;
+    case 288: chirp_rows<288>(c, filter); break;
+    case 384: chirp_rows<384>(c, filter); break;
+    case 576: chirp_rows<576>(c, filter); break;
+    case 768: chirp_rows<768>(c, filter); break;
+    case 1152: chirp_rows<1152>(c, filter); break;
+    case 1536: chirp_rows<1536>(c, filter); break;
+    case 2304: chirp_rows<2304>(c, filter); break;
+    default: chirp_rows<2048>(c, filter); break;
+  }
+}
+#undef CHIRP_POW2
+}  // namespace
+
+void launch_chirp_init(const ChirpArgs &F, double2 *tw, double2 *Y, hipStream_t s) {
+  size_t o[9];
+  chirp_offsets(F, o);
+  hipLaunchKernelGGL(k_chirp_table, dim3((F.M + 255) / 256), dim3(256), 0, s, tw + o[6], F.M);
+  const ChirpCall c = {F, nullptr, nullptr, Y, nullptr, tw + o[7], s};
+  chirp_cols_of(c, true);
+  chirp_rows_of(c, true);
+}
+
+void launch_chirp_fft(const ChirpArgs &F, const double *h0, const double *h1, double2 *Y, double2 *Z, hipStream_t s) {
+  const ChirpCall c = {F, h0, h1, Y, Z, nullptr, s};
+  chirp_cols_of(c, false);
+  chirp_rows_of(c, false);
+  chirp_back_of(c);
+}
+
+void launch_chirp_dot(const ChirpArgs &F, const double2 *Z, const double2 *data, const double *w, double2 *hw_out,
+                      double *partials, hipStream_t s) {
+  hipLaunchKernelGGL(k_chirp_dot, dim3(chirp_partials(F)), dim3(kPairThreads), 0, s, F, Z, data, w, hw_out, partials);
 }
 
 }  // namespace aak

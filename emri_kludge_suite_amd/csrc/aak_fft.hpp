@@ -53,4 +53,32 @@ constexpr long long kFinalEmpty = 0x7FF4A5A5A5A5A5B1LL;  // a signalling NaN: no
 void launch_fft_pass2_final(const FftArgs &F, const double2 *Y, double *partials, const FftFinal &fin, hipStream_t s);
 void launch_fft_final_reset(double *partials, int npairs, hipStream_t s);
 
+// Lengths N = 2M whose half has a prime factor above 13: the M-point transform as a cyclic
+// convolution of length L = R C >= 2M - 1 (Bluestein), R from 2^a, C from 2^a,
+// 3 2^a and 9 2^a.
+// Tables as in FftArgs (W_L in place of W_M); chirp: exp(-i pi m^2 / M), m < M;
+// filter: the convolution filter's transform over L, position k1 C + k2.
+struct ChirpArgs {
+  int N, M, L, R, C;
+  const double2 *twR, *twC, *twLlo, *twLhi, *twNlo, *twNhi, *chirp, *filter;
+};
+// Lengths handled (even, up to 4194304, N/2 with a prime factor above 13) and
+// the smallest R C for them.
+bool chirp_supported(int N, int *R, int *C);
+int chirp_partials(const ChirpArgs &F);
+// Size of the tables (double2 entries); the part the host fills (its size, and
+// its values when tw is given: the rest is formed by launch_chirp_init, which
+// uses L entries of Y); the pointers of F bound to a device copy.
+size_t chirp_table_size(const ChirpArgs &F);
+size_t chirp_host_tables(const ChirpArgs &F, double2 *tw);
+void chirp_bind_tables(ChirpArgs *F, double2 *tw);
+void launch_chirp_init(const ChirpArgs &F, double2 *tw, double2 *Y, hipStream_t s);
+// Channels h0 and h1 (16-byte aligned) to their M-point transforms Z ([2][M]),
+// with 2L entries of scratch Y.
+void launch_chirp_fft(const ChirpArgs &F, const double *h0, const double *h1, double2 *Y, double2 *Z, hipStream_t s);
+// chirp_partials(F) pairs (sum of <h w, d w>, sum of |h w|^2) and, if hw_out is
+// not null, the weighted spectra ([2][M+1]); data and weights in natural order.
+void launch_chirp_dot(const ChirpArgs &F, const double2 *Z, const double2 *data, const double *w, double2 *hw_out,
+                      double *partials, hipStream_t s);
+
 }  // namespace aak

@@ -215,7 +215,8 @@ class GPUAAK:
 
         fft / dot: for power-of-two lengths the column pass of the fused FFT,
         then the row pass with the weighting and both sums; otherwise the
-        rocFFT transform, then the weighted reduction.
+        transform (the library's own convolution where length/2 has a prime
+        factor above 13, else rocFFT), then the weighted reduction.
         """
         buf = np.zeros(6)
         _lib.lib().aak_get_timings(self._h, _lib.dptr(buf), 6)

@@ -49,7 +49,7 @@ int aak_test_inspiral_rates(double p, double e, double cosi, double a, double *o
  * (the handle's data and weights from aak_input_data): like[0..1] =
  * (<h|d>, <h|h>) as aak_Likelihood returns them, spec (optional) =
  * [2][length/2+1] weighted complex spectra, *fused (optional) = 1 when the
- * fused FFT ran, 0 for the rocFFT path.  Invalidates the last waveform. */
+ * fused FFT ran, 0 for the paths of other lengths.  Invalidates the last waveform. */
 struct aak_handle_s;
 int aak_test_inner_product(struct aak_handle_s *h, const double *hI, const double *hII, double *like, double *spec,
                            int *fused);
