@@ -1,8 +1,8 @@
 // aak_mlp.hip -- learned start point for the frequency map (KSParMap.cc:397-440):
 // a 4-128-128-128-3 network with GELU activations, BF16 weights and FP32
 // accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16), with its
-// training kernels (forward with saved pre-activations, backward chain,
-// weight-gradient partials, Adam) and batched inference.
+// training kernels (one for forward, backward and weight-gradient partials,
+// one for their sum and Adam) and batched inference.
 //
 // The network maps the normalised features of a trajectory point
 // (a, 1/sqrt(p), e, cos iota) to the standardised corrections
@@ -41,8 +41,10 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int H = kMlpHidden;  // 128
 constexpr int LDW = H + 8;     // LDS row stride (bf16): 272 B, conflict-free 16-byte fragment reads
-constexpr int TILE = 64;       // rows per workgroup in the forward and backward chains
-constexpr int CHUNK = 128;     // rows per workgroup in the weight-gradient partials
+constexpr int TILE = 64;       // rows per workgroup of the inference kernel
+constexpr int GROWS = 32;      // rows per tile of the gradient kernel: the K of one matrix instruction
+constexpr int LDT = GROWS + 8; // its transposed tiles' row stride (80 B, conflict-free 16-byte reads)
+constexpr int kGradGroups = 256;  // most workgroups (and partial gradients) of the gradient kernel
 constexpr int kThreads = 256;
 
 int fail(int code, const std::string &msg) { return set_last_error(code, msg); }
@@ -65,10 +67,11 @@ __device__ __forceinline__ float gelu(float z) {
   const float c = 0.7978845608028654f;
   return 0.5f * z * (1.0f + tanhf(c * (z + 0.044715f * z * z * z)));
 }
-__device__ __forceinline__ float gelu_grad(float z) {
+__device__ __forceinline__ float gelu_and_grad(float z, float *grad) {
   const float c = 0.7978845608028654f;
   const float t = tanhf(c * (z + 0.044715f * z * z * z));
-  return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * z * z);
+  *grad = 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * z * z);
+  return 0.5f * z * (1.0f + t);
 }
 
 __device__ __forceinline__ bf16x8 load8(const uint16_t *p) {
@@ -112,30 +115,19 @@ __device__ __forceinline__ void wave_gemm_128(floatx4 acc[8], const uint16_t *ac
   }
 }
 
-// ---------------------------------------------------------------- forward
-// Rows [blockIdx.x * 64, +64) of the batch; row r of the batch is row idx[r]
-// of X/T (idx null: identity).  Inference writes Y only.  Training also
-// writes the gathered inputs Xb, the pre-activations Z1..Z3 (FP32), dY and a
-// per-workgroup partial of the squared error.
-template <bool TRAIN>
-__global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restrict__ X, const float *__restrict__ T,
-                                                          const int *__restrict__ idx, int n,
+// ---------------------------------------------------------------- inference
+// Rows [blockIdx.x * 64, +64) of X to Y.
+__global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restrict__ X, int n,
                                                           const float *__restrict__ P, const uint16_t *__restrict__ Pb,
-                                                          float *__restrict__ Y, float *__restrict__ Xb,
-                                                          float *__restrict__ Z, float *__restrict__ dY,
-                                                          float *__restrict__ loss_part, float dscale) {
+                                                          float *__restrict__ Y) {
   __shared__ __align__(16) uint16_t wl[H * LDW];
   __shared__ __align__(16) uint16_t act[TILE * LDW];
   __shared__ float xs[TILE][4];
-  __shared__ float red[kThreads / 64];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int row0 = blockIdx.x * TILE;
   for (int q = threadIdx.x; q < TILE * 4; q += kThreads) {
     const int r = q >> 2, k = q & 3, gr = row0 + r;
-    float x = 0.f;
-    if (gr < n) x = X[(size_t)(idx ? idx[gr] : gr) * 4 + k];
-    xs[r][k] = x;
-    if (TRAIN && gr < n) Xb[(size_t)gr * 4 + k] = x;
+    xs[r][k] = gr < n ? X[(size_t)gr * 4 + k] : 0.f;
   }
   __syncthreads();
   // layer 1 on the VALU: lane (row l%16 of the wave, columns 32 (l/16) + j)
@@ -149,7 +141,6 @@ __global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restric
       z = fmaf(x1, bf16_to_f32(Pb[oW1 + H + c]), z);
       z = fmaf(x2, bf16_to_f32(Pb[oW1 + 2 * H + c]), z);
       z = fmaf(x3, bf16_to_f32(Pb[oW1 + 3 * H + c]), z);
-      if (TRAIN && row0 + r < n) Z[(size_t)(row0 + r) * H + c] = z;
       act[r * LDW + c] = bf16_bits(gelu(z));
     }
   }
@@ -163,13 +154,11 @@ __global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restric
     wave_gemm_128(acc, act + 16 * w * LDW, wl, H);
     __syncthreads();
     const float *bias = P + (layer ? oB3 : oB2);
-    float *Zl = TRAIN ? Z + (size_t)(layer + 1) * n * H : nullptr;
     for (int t = 0; t < 8; t++) {
       const int c = 16 * t + (l & 15);
       for (int i = 0; i < 4; i++) {
         const int r = 16 * w + 4 * (l >> 4) + i;
         const float z = acc[t][i] + bias[c];
-        if (TRAIN && row0 + r < n) Zl[(size_t)(row0 + r) * H + c] = z;
         act[r * LDW + c] = bf16_bits(gelu(z));
       }
     }
@@ -187,168 +176,325 @@ __global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restric
     const bf16x8 b = load8(wl + (l & 15) * LDW + k0 + 8 * (l >> 4));
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
   }
-  float se = 0.f;
   const int j = l & 15;
   if (j < 3) {
     for (int i = 0; i < 4; i++) {
       const int gr = row0 + 16 * w + 4 * (l >> 4) + i;
-      if (gr >= n) continue;
-      const float y = acc[i] + P[oB4 + j];
-      if (Y) Y[(size_t)gr * 3 + j] = y;
-      if (TRAIN) {
-        const float d = y - T[(size_t)(idx ? idx[gr] : gr) * 3 + j];
-        se += d * d;
-        dY[(size_t)gr * 3 + j] = dscale * d;
-      }
+      if (gr < n) Y[(size_t)gr * 3 + j] = acc[i] + P[oB4 + j];
     }
-  }
-  if (TRAIN) {
-    for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
-    if (l == 0) red[w] = se;
-    __syncthreads();
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
   }
 }
 
-// ------------------------------------------------------------ backward chain
-// dA3 = dY W4^T, dZ3 = dA3 * gelu'(Z3), dA2 = dZ3 W3^T, dZ2, dA1 = dZ2 W2^T,
-// dZ1; writes dZ1..dZ3 (FP32, [3][n][128]).
-__global__ __launch_bounds__(kThreads) void k_mlp_backward(int n, const uint16_t *__restrict__ Pb,
-                                                           const float *__restrict__ Z,
-                                                           const float *__restrict__ dY, float *__restrict__ dZ) {
-  __shared__ __align__(16) uint16_t wl[H * LDW];
-  __shared__ __align__(16) uint16_t act[TILE * LDW];
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int row0 = blockIdx.x * TILE;
-  // dY (BF16, K padded to 32) as the A operand; W4 natural (row k, outputs j)
-  for (int q = threadIdx.x; q < TILE * 32; q += kThreads) {
-    const int r = q / 32, j = q % 32, gr = row0 + r;
-    act[r * LDW + j] = (j < 3 && gr < n) ? bf16_bits(dY[(size_t)gr * 3 + j]) : (uint16_t)0;
+// ---------------------------------------------------------------- gradient
+// Forward, loss, backward chain and weight gradients of tiles of 32 rows; row r
+// of the batch is row idx[r] of X/T (idx null: identity).  A workgroup takes
+// tiles blockIdx.x, + gridDim.x, ... and writes one partial gradient and one
+// partial of the squared error.
+//   waves        wave w: rows 16 (w & 1), output columns 32 (w >> 1)
+//   products     weights as B fragments straight from L2 (Wt the transposed
+//                copies for the forward direction), the next layer's loaded while
+//                this one's activations are formed;
+//                activations and dZ through LDS, once per direction
+//   registers    gelu'(Z1..Z3) of the wave's 16 x 32 elements stay there; dW2,
+//                dW3 (K = the tile's 32 rows: one matrix instruction per
+//                16 x 16 block) and the VALU sums of dW1, dW4 and the biases
+//                accumulate over the workgroup's tiles
+// Bound by the latency of the chain of seven products and barriers, about
+// 19 us for one tile, and by the 137 KB of each partial: the work itself is
+// 0.8 GFLOP at 4096 rows.  There it takes 30 us, where separate forward,
+// backward and weight-gradient kernels took 280: those passed Z1..Z3 and
+// dZ1..dZ3 through memory, 12 MB, and the last ran 32 workgroups that walked
+// 128 rows one after another.  At 16384 rows: 43 us with up to 256 workgroups
+// (one per CU), 64 with up to 128.
+constexpr int CB = 2;              // 16-column blocks of a wave
+constexpr int kGradThreads = 512;  // eight waves: two per SIMD
+typedef bf16x8 Frags[CB][4];       // [16-column block][32-deep K step]
+__device__ __forceinline__ void load_frags(Frags f, const uint16_t *W, int l, int col0) {
+#pragma unroll
+  for (int t = 0; t < CB; t++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) f[t][k] = load8(W + (col0 + 16 * t + (l & 15)) * H + 32 * k + 8 * (l >> 4));
+}
+// acc[t] = (16 rows of act) x (the four column blocks of f)
+__device__ __forceinline__ void frag_gemm(floatx4 acc[CB], const uint16_t *act, const Frags f, int l) {
+#pragma unroll
+  for (int t = 0; t < CB; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const bf16x8 a = load8(act + (l & 15) * LDW + 32 * k + 8 * (l >> 4));
+#pragma unroll
+    for (int t = 0; t < CB; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, f[t][k], acc[t], 0, 0, 0);
   }
-  for (int q = threadIdx.x; q < H * 32; q += kThreads) {
-    const int k = q / 32, j = q % 32;
-    wl[k * LDW + j] = j < 3 ? Pb[oW4 + k * 3 + j] : (uint16_t)0;
+}
+// dW[t] += A^T dZ over the tile's rows: block row w of wave w
+__device__ __forceinline__ void grad_gemm(floatx4 acc[8], const uint16_t *at, const uint16_t *dt, int l, int w) {
+  const bf16x8 a = load8(at + (16 * w + (l & 15)) * LDT + 8 * (l >> 4));
+#pragma unroll
+  for (int t = 0; t < 8; t++) {
+    const bf16x8 d = load8(dt + (16 * t + (l & 15)) * LDT + 8 * (l >> 4));
+    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, d, acc[t], 0, 0, 0);
   }
-  __syncthreads();
-  floatx4 acc[8];
-  for (int t = 0; t < 8; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  wave_gemm_128(acc, act + 16 * w * LDW, wl, 32);
-  for (int layer = 2; layer >= 0; layer--) {
-    // acc = dA_(layer+1) in C layout: dZ = dA * gelu'(Z)
-    const float *Zl = Z + (size_t)layer * n * H;
-    float *dZl = dZ + (size_t)layer * n * H;
+}
+// Four rows r..r+3 of one column, rounded: row-major and transposed.
+__device__ __forceinline__ void put4(uint16_t *rm, uint16_t *tp, int r, int c, const float v[4]) {
+  uint16_t b[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    b[i] = bf16_bits(v[i]);
+    if (rm) rm[(r + i) * LDW + c] = b[i];
+  }
+  if (tp)
+    *reinterpret_cast<uint2 *>(tp + c * LDT + r) =
+        make_uint2(b[0] | ((uint32_t)b[1] << 16), b[2] | ((uint32_t)b[3] << 16));
+}
+
+__global__ __launch_bounds__(kGradThreads) void k_mlp_gradient(const float *__restrict__ X, const float *__restrict__ T,
+                                                              const int *__restrict__ idx, int n,
+                                                              const float *__restrict__ P,
+                                                              const uint16_t *__restrict__ Pb,
+                                                              const uint16_t *__restrict__ Wt, float *__restrict__ part,
+                                                              float *__restrict__ loss_part, float dscale) {
+  __shared__ __align__(16) uint16_t rows[5][GROWS * LDW];  // A1, A2, A3, dZ3, dZ2
+  __shared__ __align__(16) uint16_t cols[4][H * LDT];      // A1, A2, dZ3, dZ2 transposed
+  __shared__ float sm[7][H];                    // W1, b1, b2, b3
+  __shared__ __align__(16) uint16_t w4t[16 * LDW];  // W4 transposed, outputs past 3 zero
+  __shared__ __align__(16) uint16_t w4n[H * 8];     // W4, zeros past 3
+  __shared__ float xs[GROWS][4], ts[GROWS][4];
+  __shared__ float dy[8][16][4];  // each wave's rows of dY
+  __shared__ float red[2][10][H];
+  __shared__ float red4[2][4];
+  const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
+  const int rg = 16 * (w & 1), col0 = 16 * CB * (w >> 1), lc = l & 15, lr = rg + 4 * (l >> 4);
+  const int tiles = (n + GROWS - 1) / GROWS;
+
+  // the small parameters: W1 and the biases as floats, W4 for either direction
+  for (int q = tid; q < 4 * H; q += kGradThreads) sm[q / H][q % H] = bf16_to_f32(Pb[oW1 + q]);
+  for (int q = tid; q < 3 * H; q += kGradThreads) {
+    const int c = q % H, j = q / H;
+    sm[4 + j][c] = P[(j == 0 ? oB1 : j == 1 ? oB2 : oB3) + c];
+    const uint16_t v = Pb[oW4 + 3 * c + j];
+    w4t[j * LDW + c] = v;
+    w4n[c * 8 + j] = v;
+  }
+  for (int q = tid; q < 13 * H; q += kGradThreads) w4t[(3 + q / H) * LDW + q % H] = 0;
+  for (int q = tid; q < 5 * H; q += kGradThreads) w4n[(q % H) * 8 + 3 + q / H] = 0;
+  const float b4 = lc < 3 ? P[oB4 + lc] : 0.f;
+
+  floatx4 dw2[8], dw3[8];
+  float dw1[CB][4], dw4[CB][3], db1[CB], db2[CB], db3[CB], db4 = 0.f, se = 0.f;
+#pragma unroll
+  for (int t = 0; t < 8; t++) dw2[t] = dw3[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < CB; t++) {
+    db1[t] = db2[t] = db3[t] = 0.f;
+    for (int k = 0; k < 4; k++) dw1[t][k] = 0.f;
+    for (int j = 0; j < 3; j++) dw4[t][j] = 0.f;
+  }
+
+#pragma unroll 1
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const int row0 = tile * GROWS;
+    // opaque offset: keeps the weights' fragments (128 registers) from being
+    // hoisted out of the tile loop, into scratch
+    int o = 0;
+    asm volatile("" : "+s"(o));
+    Frags f;
+    load_frags(f, Wt + o, l, col0);
+    if (tid < GROWS * 4) {
+      const int r = tid >> 2, k = tid & 3, gr = row0 + r;
+      xs[r][k] = gr < n ? X[(size_t)(idx ? idx[gr] : gr) * 4 + k] : 0.f;
+    } else if (tid - GROWS * 4 < GROWS * 3) {
+      const int q = tid - GROWS * 4, r = q / 3, j = q % 3, gr = row0 + r;
+      ts[r][j] = gr < n ? T[(size_t)(idx ? idx[gr] : gr) * 3 + j] : 0.f;
+    }
     __syncthreads();
-    for (int t = 0; t < 8; t++) {
-      const int c = 16 * t + (l & 15);
+    float in[4];  // 1 for the rows below n
+#pragma unroll
+    for (int i = 0; i < 4; i++) in[i] = row0 + lr + i < n ? 1.f : 0.f;
+    float g1[CB][4], g2[CB][4], g3[CB][4];
+    // layer 1 on the VALU
+#pragma unroll
+    for (int t = 0; t < CB; t++) {
+      const int c = col0 + 16 * t + lc;
+      float v[4];
+#pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int r = 16 * w + 4 * (l >> 4) + i, gr = row0 + r;
-        float dz = 0.f;
-        if (gr < n) {
-          dz = acc[t][i] * gelu_grad(Zl[(size_t)gr * H + c]);
-          dZl[(size_t)gr * H + c] = dz;
+        const float *x = xs[lr + i];
+        float z = sm[4][c];
+        z = fmaf(x[0], sm[0][c], z);
+        z = fmaf(x[1], sm[1][c], z);
+        z = fmaf(x[2], sm[2][c], z);
+        z = fmaf(x[3], sm[3][c], z);
+        v[i] = gelu_and_grad(z, &g1[t][i]);
+      }
+      put4(rows[0], cols[0], lr, c, v);
+    }
+    __syncthreads();
+    floatx4 acc[CB];
+    frag_gemm(acc, rows[0] + rg * LDW, f, l);
+    load_frags(f, Wt + o + H * H, l, col0);
+#pragma unroll
+    for (int t = 0; t < CB; t++) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = gelu_and_grad(acc[t][i] + sm[5][col0 + 16 * t + lc], &g2[t][i]);
+      put4(rows[1], cols[1], lr, col0 + 16 * t + lc, v);
+    }
+    __syncthreads();
+    frag_gemm(acc, rows[1] + rg * LDW, f, l);
+    load_frags(f, Pb + o + oW3, l, col0);
+#pragma unroll
+    for (int t = 0; t < CB; t++) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = gelu_and_grad(acc[t][i] + sm[6][col0 + 16 * t + lc], &g3[t][i]);
+      put4(rows[2], nullptr, lr, col0 + 16 * t + lc, v);
+    }
+    __syncthreads();
+    // layer 4 and the loss, by all four waves of the rows
+    {
+      floatx4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bf16x8 a = load8(rows[2] + (rg + lc) * LDW + 32 * k + 8 * (l >> 4));
+        y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, load8(w4t + lc * LDW + 32 * k + 8 * (l >> 4)), y, 0, 0, 0);
+      }
+      if (lc < 3) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float d = row0 + lr + i < n ? y[i] + b4 - ts[lr + i][lc] : 0.f;
+          se += d * d;
+          db4 += dscale * d;
+          dy[w][4 * (l >> 4) + i][lc] = dscale * d;
         }
-        act[r * LDW + c] = bf16_bits(dz);
       }
     }
-    if (layer == 0) break;
-    stage_hxh(wl, Pb + (layer == 2 ? oW3 : oW2), false);
     __syncthreads();
-    for (int t = 0; t < 8; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    wave_gemm_128(acc, act + 16 * w * LDW, wl, H);
+    // dA3 = dY W4^T (K padded from 3); dZ = dA * gelu'(Z)
+    {
+      uint16_t u[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (l < 16)
+        for (int q = 0; q < 3; q++) u[q] = bf16_bits(dy[w][lc][q]);
+      bf16x8 a;
+      __builtin_memcpy(&a, u, 16);
+#pragma unroll
+      for (int t = 0; t < CB; t++) {
+        // lanes past 15 face the zeros of dY's K = 8..31
+        const bf16x8 b = load8(w4n + (col0 + 16 * t + lc) * 8);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < CB; t++) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        v[i] = in[i] != 0.f ? acc[t][i] * g3[t][i] : 0.f;
+        db3[t] += v[i];
+        const float a3 = bf16_to_f32(rows[2][(lr + i) * LDW + col0 + 16 * t + lc]);
+        const float *d = dy[w][4 * (l >> 4) + i];
+#pragma unroll
+        for (int j = 0; j < 3; j++) dw4[t][j] = fmaf(a3, d[j], dw4[t][j]);
+      }
+      put4(rows[3], cols[2], lr, col0 + 16 * t + lc, v);
+    }
+    __syncthreads();
+    frag_gemm(acc, rows[3] + rg * LDW, f, l);
+    load_frags(f, Pb + o + oW2, l, col0);
+#pragma unroll
+    for (int t = 0; t < CB; t++) {
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        v[i] = in[i] != 0.f ? acc[t][i] * g2[t][i] : 0.f;
+        db2[t] += v[i];
+      }
+      put4(rows[4], cols[3], lr, col0 + 16 * t + lc, v);
+    }
+    __syncthreads();
+    frag_gemm(acc, rows[4] + rg * LDW, f, l);
+#pragma unroll
+    for (int t = 0; t < CB; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float d = in[i] != 0.f ? acc[t][i] * g1[t][i] : 0.f;
+        db1[t] += d;
+#pragma unroll
+        for (int k = 0; k < 4; k++) dw1[t][k] = fmaf(xs[lr + i][k], d, dw1[t][k]);
+      }
+    grad_gemm(dw3, cols[1], cols[2], l, w);
+    grad_gemm(dw2, cols[0], cols[3], l, w);
+    __syncthreads();  // the next tile overwrites
   }
-}
 
-// ------------------------------------------------------- weight gradients
-// Partial gradients over rows [blockIdx.x * 128, +128): dW2 = A1^T dZ2 and
-// dW3 = A2^T dZ3 on the matrix cores (A = bf16(gelu(Z)), dZ rounded to BF16),
-// dW1 = X^T dZ1, dW4 = A3^T dY and the bias sums on the VALU.
-__global__ __launch_bounds__(kThreads) void k_mlp_wgrad(int n, const float *__restrict__ Xb,
-                                                        const float *__restrict__ Z, const float *__restrict__ dZ,
-                                                        const float *__restrict__ dY, float *__restrict__ part) {
-  __shared__ __align__(16) uint16_t at[H * LDW];  // A^T: row = feature m, rows of the chunk contiguous
-  __shared__ __align__(16) uint16_t dt[H * LDW];  // dZ^T
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int row0 = blockIdx.x * CHUNK;
-  const int rows = min(CHUNK, n - row0);
   float *out = part + (size_t)blockIdx.x * kNP;
-  for (int m = 0; m < 2; m++) {  // m = 0: dW2 (A1, dZ2), m = 1: dW3 (A2, dZ3)
-    const float *Zs = Z + (size_t)m * n * H;
-    const float *dZs = dZ + (size_t)(m + 1) * n * H;
-    __syncthreads();
-    for (int q = threadIdx.x; q < CHUNK * H; q += kThreads) {
-      const int r = q / H, c = q % H;
-      uint16_t a = 0, d = 0;
-      if (r < rows) {
-        a = bf16_bits(gelu(Zs[(size_t)(row0 + r) * H + c]));
-        d = bf16_bits(dZs[(size_t)(row0 + r) * H + c]);
-      }
-      at[c * LDW + r] = a;
-      dt[c * LDW + r] = d;
+#pragma unroll
+  for (int t = 0; t < 8; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int q = (16 * w + 4 * (l >> 4) + i) * H + 16 * t + lc;
+      out[oW2 + q] = dw2[t][i];
+      out[oW3 + q] = dw3[t][i];
     }
-    __syncthreads();
-    // 8 x 8 output tiles of 16 x 16; wave w takes tile rows 2w, 2w + 1
-    for (int tr = 2 * w; tr < 2 * w + 2; tr++) {
-      floatx4 acc[8];
-      for (int t = 0; t < 8; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-      wave_gemm_128(acc, at + 16 * tr * LDW, dt, CHUNK);
-      float *dW = out + (m ? oW3 : oW2);
-      for (int t = 0; t < 8; t++)
-        for (int i = 0; i < 4; i++) dW[(16 * tr + 4 * (l >> 4) + i) * H + 16 * t + (l & 15)] = acc[t][i];
+  // the VALU sums: over a column's lanes, then the two row groups.  Sum s:
+  // 0..3 dW1, 4..6 dW4, 7..9 the biases 1..3
+  auto rowsum = [](float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+  };
+#pragma unroll
+  for (int t = 0; t < CB; t++)
+#pragma unroll
+    for (int s = 0; s < 10; s++) {
+      const float x = rowsum(s < 4 ? dw1[t][s] : s < 7 ? dw4[t][s - 4] : s == 7 ? db1[t] : s == 8 ? db2[t] : db3[t]);
+      if (l < 16) red[w & 1][s][col0 + 16 * t + lc] = x;
     }
+  se = rowsum(se);
+  db4 = rowsum(db4);
+  if (w < 2 && l < 3) red4[w][l] = db4;
+  se += __shfl_xor(se, 1);  // lanes 0..2 hold the sums, the rest 0
+  se += __shfl_xor(se, 2);
+  if (w < 2 && l == 0) red4[w][3] = se;
+  __syncthreads();
+  for (int q = tid; q < 10 * H; q += kGradThreads) {
+    const int s = q / H, c = q % H;
+    const int o = s < 4 ? oW1 + s * H + c : s < 7 ? oW4 + 3 * c + s - 4 : s == 7 ? oB1 + c : s == 8 ? oB2 + c : oB3 + c;
+    out[o] = red[0][s][c] + red[1][s][c];
   }
-  // dW1[k][c] = sum_r X[r][k] dZ1[r][c]; db_l[c] = sum_r dZ_l[r][c]
-  for (int c = threadIdx.x; c < H; c += kThreads) {
-    float g0 = 0.f, g1 = 0.f, g2 = 0.f, g3 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    for (int r = 0; r < rows; r++) {
-      const size_t gr = row0 + r;
-      const float d1 = dZ[gr * H + c];
-      g0 = fmaf(Xb[gr * 4 + 0], d1, g0);
-      g1 = fmaf(Xb[gr * 4 + 1], d1, g1);
-      g2 = fmaf(Xb[gr * 4 + 2], d1, g2);
-      g3 = fmaf(Xb[gr * 4 + 3], d1, g3);
-      s1 += d1;
-      s2 += dZ[(size_t)n * H + gr * H + c];
-      s3 += dZ[(size_t)2 * n * H + gr * H + c];
-    }
-    out[oW1 + c] = g0;
-    out[oW1 + H + c] = g1;
-    out[oW1 + 2 * H + c] = g2;
-    out[oW1 + 3 * H + c] = g3;
-    out[oB1 + c] = s1;
-    out[oB2 + c] = s2;
-    out[oB3 + c] = s3;
-  }
-  // dW4[k][j] = sum_r A3[r][k] dY[r][j] (A3 = bf16(gelu(Z3))); db4
-  for (int q = threadIdx.x; q < 3 * H + 3; q += kThreads) {
-    float g = 0.f;
-    if (q < 3 * H) {
-      const int k = q / 3, j = q % 3;
-      for (int r = 0; r < rows; r++) {
-        const size_t gr = row0 + r;
-        g = fmaf(bf16_to_f32(bf16_bits(gelu(Z[(size_t)2 * n * H + gr * H + k]))), dY[gr * 3 + j], g);
-      }
-      out[oW4 + q] = g;
-    } else {
-      const int j = q - 3 * H;
-      for (int r = 0; r < rows; r++) g += dY[(size_t)(row0 + r) * 3 + j];
-      out[oB4 + j] = g;
-    }
-  }
+  if (tid < 3) out[oB4 + tid] = red4[0][tid] + red4[1][tid];
+  if (tid == 3) loss_part[blockIdx.x] = red4[0][3] + red4[1][3];
 }
 
 // ----------------------------------------------------------------- Adam
-// g = sum of the chunk partials; with step > 0 an Adam step on the FP32
-// master copy, whose BF16 copy is refreshed; with step == 0 only g is written.
-__global__ __launch_bounds__(kThreads) void k_mlp_adam(int nchunks, const float *__restrict__ part,
+// g = sum of the partials (four slices of them per parameter, 64 parameters per
+// workgroup, so that many loads are in flight); with step > 0 an Adam step on
+// the FP32 master copy, whose BF16 copies are refreshed; with step == 0 only g
+// is written.
+__device__ __forceinline__ void put_bf16(int p, float x, uint16_t *Pb, uint16_t *Wt) {
+  const uint16_t b = bf16_bits(x);
+  Pb[p] = b;
+  const int q2 = p - oW2, q3 = p - oW3;
+  if (q2 >= 0 && q2 < H * H) Wt[(q2 % H) * H + q2 / H] = b;
+  if (q3 >= 0 && q3 < H * H) Wt[H * H + (q3 % H) * H + q3 / H] = b;
+}
+
+__global__ __launch_bounds__(kThreads) void k_mlp_adam(int nparts, const float *__restrict__ part,
                                                        float *__restrict__ grad, float *__restrict__ P,
-                                                       uint16_t *__restrict__ Pb, float *__restrict__ m1,
-                                                       float *__restrict__ m2, int step, float lr, float b1,
-                                                       float b2, float eps) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p >= kNP) return;
+                                                       uint16_t *__restrict__ Pb, uint16_t *__restrict__ Wt,
+                                                       float *__restrict__ m1, float *__restrict__ m2, int step,
+                                                       float lr, float b1, float b2, float eps) {
+  __shared__ float sum[4][64];
+  const int j = threadIdx.x & 63, slice = threadIdx.x >> 6, p = blockIdx.x * 64 + j;
   float g = 0.f;
-  for (int c = 0; c < nchunks; c++) g += part[(size_t)c * kNP + p];
-  if (grad) grad[p] = g;
+  if (p < kNP) {
+#pragma unroll 8
+    for (int c = slice; c < nparts; c += 4) g += part[(size_t)c * kNP + p];
+  }
+  sum[slice][j] = g;
+  __syncthreads();
+  if (slice || p >= kNP) return;
+  g = (sum[0][j] + sum[1][j]) + (sum[2][j] + sum[3][j]);
+  grad[p] = g;
   if (step <= 0) return;
   const float a = b1 * m1[p] + (1.f - b1) * g, v = b2 * m2[p] + (1.f - b2) * g * g;
   m1[p] = a;
@@ -356,12 +502,12 @@ __global__ __launch_bounds__(kThreads) void k_mlp_adam(int nchunks, const float 
   const float ah = a / (1.f - powf(b1, (float)step)), vh = v / (1.f - powf(b2, (float)step));
   const float x = P[p] - lr * ah / (sqrtf(vh) + eps);
   P[p] = x;
-  Pb[p] = bf16_bits(x);
+  put_bf16(p, x, Pb, Wt);
 }
 
-__global__ void k_mlp_round(const float *__restrict__ P, uint16_t *__restrict__ Pb) {
+__global__ void k_mlp_round(const float *__restrict__ P, uint16_t *__restrict__ Pb, uint16_t *__restrict__ Wt) {
   const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p < kNP) Pb[p] = bf16_bits(P[p]);
+  if (p < kNP) put_bf16(p, P[p], Pb, Wt);
 }
 
 }  // namespace
@@ -370,14 +516,14 @@ __global__ void k_mlp_round(const float *__restrict__ P, uint16_t *__restrict__ 
 struct aak_mlp_s {
   float *P = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
   uint16_t *Pb = nullptr;
+  uint16_t *Wt = nullptr;  // W2, W3 in BF16, transposed (row n holds input k)
   int step = 0;
   float norm[kMlpNorm] = {};  // feature centres/scales and target means/scales
   hipStream_t s = nullptr;
   int dev = 0;  // device the model lives on (callers may be other host threads)
   // training / gradient scratch (grown on demand)
   int cap = 0;
-  float *X = nullptr, *T = nullptr, *Xb = nullptr, *Z = nullptr, *dZ = nullptr, *dY = nullptr, *loss = nullptr,
-        *part = nullptr;
+  float *X = nullptr, *T = nullptr, *loss = nullptr, *part = nullptr;
   int *idx = nullptr;
   int data_n = 0;
   // inference scratch
@@ -391,29 +537,29 @@ struct aak_mlp_s {
 namespace aak {
 
 static void free_scratch(aak_mlp_s *m) {
-  void *ps[] = {m->X, m->T, m->Xb, m->Z, m->dZ, m->dY, m->loss, m->part, m->idx};
+  void *ps[] = {m->X, m->T, m->loss, m->part, m->idx};
   for (void *p : ps)
     if (p) (void)hipFree(p);
-  m->X = m->T = m->Xb = m->Z = m->dZ = m->dY = m->loss = m->part = nullptr;
+  m->X = m->T = m->loss = m->part = nullptr;
   m->idx = nullptr;
   m->cap = 0;
   m->data_n = 0;
 }
 
+static int grad_groups(int B) { return std::min(kGradGroups, (B + GROWS - 1) / GROWS); }
+
 // Scratch for batches of up to B rows over a data set of `data` rows.
 static int grow_scratch(aak_mlp_s *m, int B, int data) {
-  if (B > m->cap) {
-    void *ps[] = {m->Xb, m->Z, m->dZ, m->dY, m->loss, m->part};
+  const int groups = grad_groups(B);
+  if (groups > m->cap) {
+    void *ps[] = {m->loss, m->part};
     for (void *p : ps)
       if (p) (void)hipFree(p);
-    const int tiles = (B + TILE - 1) / TILE, chunks = (B + CHUNK - 1) / CHUNK;
-    MLPCHK(hipMalloc(&m->Xb, sizeof(float) * 4 * (size_t)B));
-    MLPCHK(hipMalloc(&m->Z, sizeof(float) * 3 * (size_t)B * H));
-    MLPCHK(hipMalloc(&m->dZ, sizeof(float) * 3 * (size_t)B * H));
-    MLPCHK(hipMalloc(&m->dY, sizeof(float) * 3 * (size_t)B));
-    MLPCHK(hipMalloc(&m->loss, sizeof(float) * tiles));
-    MLPCHK(hipMalloc(&m->part, sizeof(float) * (size_t)chunks * kNP));
-    m->cap = B;
+    m->loss = m->part = nullptr;
+    m->cap = 0;
+    MLPCHK(hipMalloc(&m->loss, sizeof(float) * groups));
+    MLPCHK(hipMalloc(&m->part, sizeof(float) * (size_t)groups * kNP));
+    m->cap = groups;
   }
   if (data > m->data_n) {
     if (m->X) (void)hipFree(m->X);
@@ -427,22 +573,21 @@ static int grow_scratch(aak_mlp_s *m, int B, int data) {
   return 0;
 }
 
-// One forward + backward over rows idx[off .. off+B) of the uploaded data;
+// One forward + backward over rows idx[0 .. B) of the uploaded data (idx null:
+// its first B);
 // with step > 0 an Adam update.  loss_sum (optional) gets the squared error.
-static int train_step(aak_mlp_s *m, int off, int B, float lr, bool update, double *loss_sum) {
-  const int tiles = (B + TILE - 1) / TILE, chunks = (B + CHUNK - 1) / CHUNK;
+static int train_step(aak_mlp_s *m, const int *idx, int B, float lr, bool update, double *loss_sum) {
+  const int groups = grad_groups(B);
   const float dscale = 2.f / (3.f * (float)B);
-  hipLaunchKernelGGL(k_mlp_forward<true>, dim3(tiles), dim3(kThreads), 0, m->s, m->X, m->T, m->idx + off, B, m->P,
-                     m->Pb, nullptr, m->Xb, m->Z, m->dY, m->loss, dscale);
-  hipLaunchKernelGGL(k_mlp_backward, dim3(tiles), dim3(kThreads), 0, m->s, B, m->Pb, m->Z, m->dY, m->dZ);
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(chunks), dim3(kThreads), 0, m->s, B, m->Xb, m->Z, m->dZ, m->dY, m->part);
+  hipLaunchKernelGGL(k_mlp_gradient, dim3(groups), dim3(kGradThreads), 0, m->s, m->X, m->T, idx, B, m->P, m->Pb, m->Wt,
+                     m->part, m->loss, dscale);
   if (update) m->step++;
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kNP + kThreads - 1) / kThreads), dim3(kThreads), 0, m->s, chunks, m->part,
-                     m->grad, m->P, m->Pb, m->m1, m->m2, update ? m->step : 0, lr, 0.9f, 0.999f, 1e-8f);
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kNP + 63) / 64), dim3(kThreads), 0, m->s, groups, m->part, m->grad, m->P, m->Pb,
+                     m->Wt, m->m1, m->m2, update ? m->step : 0, lr, 0.9f, 0.999f, 1e-8f);
   MLPCHK(hipGetLastError());
   if (loss_sum) {
-    std::vector<float> lp(tiles);
-    MLPCHK(hipMemcpyAsync(lp.data(), m->loss, sizeof(float) * tiles, hipMemcpyDeviceToHost, m->s));
+    std::vector<float> lp(groups);
+    MLPCHK(hipMemcpyAsync(lp.data(), m->loss, sizeof(float) * groups, hipMemcpyDeviceToHost, m->s));
     MLPCHK(hipStreamSynchronize(m->s));
     double s = 0.0;
     for (float x : lp) s += x;
@@ -476,8 +621,8 @@ int mlp_infer(aak_mlp_s *m, const double *pts, int n, double *maps) {
   m->hy.resize(3 * (size_t)n);
   for (int i = 0; i < n; i++) features(m, pts + 4 * (size_t)i, m->hx.data() + 4 * (size_t)i);
   MLPCHK(hipMemcpyAsync(m->iX, m->hx.data(), sizeof(float) * 4 * (size_t)n, hipMemcpyHostToDevice, m->s));
-  hipLaunchKernelGGL(k_mlp_forward<false>, dim3((n + TILE - 1) / TILE), dim3(kThreads), 0, m->s, m->iX, nullptr,
-                     nullptr, n, m->P, m->Pb, m->iY, nullptr, nullptr, nullptr, nullptr, 0.f);
+  hipLaunchKernelGGL(k_mlp_forward, dim3((n + TILE - 1) / TILE), dim3(kThreads), 0, m->s, m->iX, n, m->P, m->Pb,
+                     m->iY);
   MLPCHK(hipGetLastError());
   MLPCHK(hipMemcpyAsync(m->hy.data(), m->iY, sizeof(float) * 3 * (size_t)n, hipMemcpyDeviceToHost, m->s));
   MLPCHK(hipStreamSynchronize(m->s));
@@ -520,7 +665,9 @@ int aak_mlp_create(int seed, aak_mlp *out) {
   m->m1 = bufs[1];
   m->m2 = bufs[2];
   m->grad = bufs[3];
-  if (hipMalloc(&m->Pb, sizeof(uint16_t) * kNP) != hipSuccess) return bail(fail(-100, "device allocation failed"));
+  if (hipMalloc(&m->Pb, sizeof(uint16_t) * kNP) != hipSuccess ||
+      hipMalloc(&m->Wt, sizeof(uint16_t) * 2 * H * H) != hipSuccess)
+    return bail(fail(-100, "device allocation failed"));
   // He-style initialisation; identity normalisation until the trainer sets it
   std::mt19937_64 rng((uint64_t)seed);
   std::vector<float> p(kNP, 0.f);
@@ -548,7 +695,7 @@ int aak_mlp_destroy(aak_mlp m) {
   if (!m) return fail(-1, "null model");
   if (m->s) (void)hipStreamSynchronize(m->s);
   free_scratch(m);
-  void *ps[] = {m->P, m->m1, m->m2, m->grad, m->Pb, m->iX, m->iY};
+  void *ps[] = {m->P, m->m1, m->m2, m->grad, m->Pb, m->Wt, m->iX, m->iY};
   for (void *p : ps)
     if (p) (void)hipFree(p);
   if (m->s) (void)hipStreamDestroy(m->s);
@@ -559,7 +706,7 @@ int aak_mlp_destroy(aak_mlp m) {
 int aak_mlp_set_params(aak_mlp m, const float *params, const float *norm) {
   if (!m || !params) return fail(-2, "null argument");
   MLPCHK(hipMemcpyAsync(m->P, params, sizeof(float) * kNP, hipMemcpyHostToDevice, m->s));
-  hipLaunchKernelGGL(k_mlp_round, dim3((kNP + kThreads - 1) / kThreads), dim3(kThreads), 0, m->s, m->P, m->Pb);
+  hipLaunchKernelGGL(k_mlp_round, dim3((kNP + kThreads - 1) / kThreads), dim3(kThreads), 0, m->s, m->P, m->Pb, m->Wt);
   MLPCHK(hipGetLastError());
   MLPCHK(hipStreamSynchronize(m->s));
   if (norm) std::memcpy(m->norm, norm, sizeof(m->norm));
@@ -592,8 +739,8 @@ int aak_mlp_forward(aak_mlp m, const float *X, int n, float *Y) {
     m->icap = n;
   }
   MLPCHK(hipMemcpyAsync(m->iX, X, sizeof(float) * 4 * (size_t)n, hipMemcpyHostToDevice, m->s));
-  hipLaunchKernelGGL(k_mlp_forward<false>, dim3((n + TILE - 1) / TILE), dim3(kThreads), 0, m->s, m->iX, nullptr,
-                     nullptr, n, m->P, m->Pb, m->iY, nullptr, nullptr, nullptr, nullptr, 0.f);
+  hipLaunchKernelGGL(k_mlp_forward, dim3((n + TILE - 1) / TILE), dim3(kThreads), 0, m->s, m->iX, n, m->P, m->Pb,
+                     m->iY);
   MLPCHK(hipGetLastError());
   MLPCHK(hipMemcpyAsync(Y, m->iY, sizeof(float) * 3 * (size_t)n, hipMemcpyDeviceToHost, m->s));
   MLPCHK(hipStreamSynchronize(m->s));
@@ -605,13 +752,10 @@ int aak_mlp_gradient(aak_mlp m, const float *X, const float *T, int n, float *gr
   MLPCHK(hipSetDevice(m->dev));
   int rc = grow_scratch(m, n, n);
   if (rc) return rc;
-  std::vector<int> id(n);
-  for (int i = 0; i < n; i++) id[i] = i;
   MLPCHK(hipMemcpyAsync(m->X, X, sizeof(float) * 4 * (size_t)n, hipMemcpyHostToDevice, m->s));
   MLPCHK(hipMemcpyAsync(m->T, T, sizeof(float) * 3 * (size_t)n, hipMemcpyHostToDevice, m->s));
-  MLPCHK(hipMemcpyAsync(m->idx, id.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice, m->s));
   double ls = 0.0;
-  rc = train_step(m, 0, n, 0.f, false, &ls);
+  rc = train_step(m, nullptr, n, 0.f, false, &ls);
   if (rc) return rc;
   MLPCHK(hipMemcpyAsync(grad, m->grad, sizeof(float) * kNP, hipMemcpyDeviceToHost, m->s));
   MLPCHK(hipStreamSynchronize(m->s));
@@ -644,7 +788,7 @@ int aak_mlp_train(aak_mlp m, const float *X, const float *T, int n, int epochs, 
       const double f = 0.5 * (1.0 + cos(M_PI * (double)done / (double)total));
       const float lr = (float)(lr1 + (lr0 - lr1) * f);
       double ls = 0.0;
-      rc = train_step(m, st * batch, batch, lr, true, (st == steps_per_epoch - 1) ? &ls : nullptr);
+      rc = train_step(m, m->idx + (size_t)st * batch, batch, lr, true, (st == steps_per_epoch - 1) ? &ls : nullptr);
       if (rc) return rc;
       ep_loss = ls / (3.0 * batch);
     }
