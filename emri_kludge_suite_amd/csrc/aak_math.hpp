@@ -195,7 +195,8 @@ struct Carlson {
 // transcribed from the reference's device copies (kernel.cu:163-230); the
 // oracle transcribes the host copies (KSParMap.cc:146-209).
 struct PN {
-  AAK_HD static double dtdm(double v, double e, double Y, double q) {
+  // numerators of the maps below
+  AAK_HD static double dtdm_num(double v, double e, double Y, double q) {
     const double v2 = v * v, v3 = v2 * v, v4 = v2 * v2, e2 = e * e, e4 = e2 * e2, Y2 = Y * Y, q2 = q * q;
     return (2. * e4 * (240. + v2 * (-120. + v * (42. * (-27. + 4. * q2) * v + (-6567. + 1996. * q2) * v3 +
                                                  48. * q * (8. + 77. * v2) * Y - 4. * q2 * v * (90. + 1577. * v2) * Y2))) +
@@ -205,33 +206,39 @@ struct PN {
             8. * e2 * (-48. + v2 * (8. - 64. * q * v * Y - 688. * q * v3 * Y +
                                     2. * v2 * (99. + 16. * q2 * (-1. + 2. * Y2)) + v4 * (1233. + 8. * q2 * (-47. + 150. * Y2)))) +
             16. * (16. + v2 * (24. + v2 * (27. * (2. + 5. * v2) - 48. * q * v * Y +
-                                           4. * q2 * (2. - v2 + (-2. + 3. * v2) * Y2))))) / (256. * v4);
+                                           4. * q2 * (2. - v2 + (-2. + 3. * v2) * Y2)))));
   }
-  AAK_HD static double drdm(double v, double e, double Y, double q) {
+  AAK_HD static double drdm_num(double v, double e, double Y, double q) {
     const double v2 = v * v, v3 = v2 * v, e2 = e * e, e4 = e2 * e2, Y2 = Y * Y, q2 = q * q;
     return (16. + 8. * (-3. + e2) * v2 - 16. * (-3. + e2) * q * v3 * Y +
             8. * (33. + 4. * e2 - 3. * e4) * q * v3 * v2 * Y +
             v3 * v3 * (-351. + 132. * q2 + e2 * (-135. + 21. * e2 + 5. * e4 + 2. * (7. + e2) * q2) +
                        2. * (-204. + 13. * e2 * (-3. + e2)) * q2 * Y2) +
-            2. * v2 * v2 * (-45. + 3. * e4 + 4. * q2 * (1. - 4. * Y2) + 2. * e2 * q2 * (1. + Y2))) / (16. * v);
+            2. * v2 * v2 * (-45. + 3. * e4 + 4. * q2 * (1. - 4. * Y2) + 2. * e2 * q2 * (1. + Y2)));
   }
-  AAK_HD static double dthetadm(double v, double e, double Y, double q) {
+  AAK_HD static double dthetadm_num(double v, double e, double Y, double q) {
     const double v2 = v * v, v3 = v2 * v, e2 = e * e, e4 = e2 * e2, Y2 = Y * Y, q2 = q * q;
     return (16. + 8. * (3. + e2) * v2 - 16. * (3. + e2) * q * v3 * Y -
             8. * (3. + e2) * (5. + 3. * e2) * q * v3 * v2 * Y +
             v3 * v3 * (135. - 54. * q2 + e2 * (5. * (27. + 9. * e2 + e4) + 2. * (-38. + e2) * q2) +
                        2. * (57. + 90. * e2 + 13. * e4) * q2 * Y2) +
-            2. * v2 * v2 * (27. + 3. * e4 + 2. * q2 * (-1. + 7. * Y2) + 2. * e2 * (9. + q2 * (1. + Y2)))) / (16. * v);
+            2. * v2 * v2 * (27. + 3. * e4 + 2. * q2 * (-1. + 7. * Y2) + 2. * e2 * (9. + q2 * (1. + Y2))));
   }
-  AAK_HD static double dphidm(double v, double e, double Y, double q) {
+  AAK_HD static double dphidm_num(double v, double e, double Y, double q) {
     const double v2 = v * v, v3 = v2 * v, e2 = e * e, e4 = e2 * e2, Y2 = Y * Y, q2 = q * q;
     return (16. + 8. * (3. + e2) * v2 - 16. * q * v3 * (-2. + (3. + e2) * Y) -
             8. * q * v3 * v2 * (-6. + 15. * Y + 3. * e4 * Y + 2. * e2 * (-4. + 7. * Y)) +
             2. * v2 * v2 * (27. + 3. * e4 + 2. * q2 * (-1. + Y) * (1. + 7. * Y) + 2. * e2 * (9. + q2 * (1. + Y2))) +
             v3 * v3 * (5. * e4 * e2 + e4 * (45. + q2 * (2. + 26. * Y2)) +
-                       e2 * (135. + 4. * q2 * (-19. + 5. * Y * (-7. + 9. * Y))) + 3. * (45. + 2. * q2 * (-9. + Y * (-6. + 19. * Y))))) /
-           (16. * v);
+                       e2 * (135. + 4. * q2 * (-19. + 5. * Y * (-7. + 9. * Y))) + 3. * (45. + 2. * q2 * (-9. + Y * (-6. + 19. * Y)))));
   }
+  AAK_HD static double dtdm(double v, double e, double Y, double q) {
+    const double v2 = v * v;
+    return dtdm_num(v, e, Y, q) / (256. * (v2 * v2));
+  }
+  AAK_HD static double drdm(double v, double e, double Y, double q) { return drdm_num(v, e, Y, q) / (16. * v); }
+  AAK_HD static double dthetadm(double v, double e, double Y, double q) { return dthetadm_num(v, e, Y, q) / (16. * v); }
+  AAK_HD static double dphidm(double v, double e, double Y, double q) { return dphidm_num(v, e, Y, q) / (16. * v); }
   // |Omega_phi| of the AK orbit, prograde or retrograde (gpuAAK.cc:17-26).
   AAK_HD static double omega_phi(double v, double e, double cosi, double s, double M) {
     if (cosi > 0) return dphidm(v, e, cosi, s) / dtdm(v, e, cosi, s) / M;
