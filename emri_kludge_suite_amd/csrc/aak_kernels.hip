@@ -2231,10 +2231,10 @@ __device__ inline double harmonic_phase(const DenseParams &P, const SampleGeom &
 constexpr int kMsThreads = 256;
 constexpr int kTaylorModes = 128;
 // Samples per expansion block: 256 << exp_shift (host-set, default 2 in the
-// mixed form and 0 in FP64).  The mixed form's looser order bound lets one
-// expansion serve 1024 samples (the mean order rises from 2.0 to 2.5 over the
-// production prior while the setup work falls fourfold); FP64 keeps 256,
-// where wider blocks would send more of them to the per-sample path.
+// mixed form and in FP64 from 2^18 samples on, else 0).  One expansion serves
+// 1024 samples while the setup work falls fourfold and the mean order rises
+// little (mixed, over the production prior: from 2.0 to 2.5); blocks that need
+// more than order 8 are expanded per 256 samples.
 __host__ __device__ inline int exp_shift(const DenseParams &P) { return P.xshift; }
 constexpr int kSetupThreads = 64;
 // doubles reserved per block in B.ms_coef per harmonic (orders up to kTaylorMax)
