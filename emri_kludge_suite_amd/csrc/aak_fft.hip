@@ -211,28 +211,49 @@ __device__ __forceinline__ void fft_conj_product(double2 *x, int t, const double
   fft_stages<L, NT, RS>(x, t, tw);
 }
 
-// Whole L-point FFT whose first stage (no twiddles) reads straight from global
-// memory: butterfly j reads src[j + r L / RS], contiguous across the threads
-// for each r.
+// The points of a thread's first-stage butterflies, straight from global memory
+// (a caller requests them before what it needs only after the FFT: loads return
+// in order; at N = 2^18 the second pass takes 12.0 us so, 15.4 with them last):
+// butterfly j reads src[j + r L / RS], contiguous across the threads for each r.
 template <int L, int NT>
-__device__ __forceinline__ void fft_first_global(const double2 *src, double2 *x, int t, const double2 *tw) {
-  constexpr int RS = stage_radix(L);
-  constexpr int NB = L / RS;
-  constexpr int PER = (NB + NT - 1) / NT;
+struct FirstPoints {
+  static constexpr int RS = stage_radix(L), NB = L / RS, PER = (NB + NT - 1) / NT;
+  double2 v[PER][RS];
+  __device__ __forceinline__ void load(const double2 *src, int t) {
 #pragma unroll
-  for (int u = 0; u < PER; u++) {
+    for (int u = 0; u < PER; u++) {
+      const int j = t + u * NT;
+      if (NB % NT == 0 || j < NB) {
+#pragma unroll
+        for (int r = 0; r < RS; r++) v[u][r] = src[j + r * NB];
+      }
+    }
+  }
+};
+
+// Whole L-point FFT from the points of the first stage (no twiddles).
+template <int L, int NT>
+__device__ __forceinline__ void fft_first(FirstPoints<L, NT> &p, double2 *x, int t, const double2 *tw) {
+  constexpr int RS = FirstPoints<L, NT>::RS, NB = FirstPoints<L, NT>::NB;
+#pragma unroll
+  for (int u = 0; u < FirstPoints<L, NT>::PER; u++) {
     const int j = t + u * NT;
     if (NB % NT == 0 || j < NB) {
-      double2 v[RS], o[RS];
-#pragma unroll
-      for (int r = 0; r < RS; r++) v[r] = src[j + r * NB];
-      dft<RS>(v, o);
+      double2 o[RS];
+      dft<RS>(p.v[u], o);
 #pragma unroll
       for (int r = 0; r < RS; r++) x[pad(j * RS + r)] = o[r];
     }
   }
   __syncthreads();
   fft_stages<L, NT, RS>(x, t, tw);
+}
+
+template <int L, int NT>
+__device__ __forceinline__ void fft_first_global(const double2 *src, double2 *x, int t, const double2 *tw) {
+  FirstPoints<L, NT> p;
+  p.load(src, t);
+  fft_first<L, NT>(p, x, t, tw);
 }
 
 __device__ inline double2 tw2(const double2 *hi, const double2 *lo, long long e) {
@@ -424,8 +445,11 @@ __global__ __launch_bounds__(2 * fft_threads<LC>()) void k_fft_rows(FftArgs F, c
   const double2 *Yc = Y + (size_t)ch * F.M;
   const double2 *Dp = F.Dp[ch];
   const double *wp = F.wp[ch];
-  // this thread's weighted data and weights, fetched before the FFT so their
-  // latency hides behind it; k2 = tid + q 2NT in rows A and B
+  // the FFT's points, then this thread's weighted data and weights, whose
+  // latency hides behind the FFT (loads return in order, so the points come
+  // first); k2 = tid + q 2NT in rows A and B
+  FirstPoints<LC, NT> points;
+  points.load(Yc + (size_t)(half ? B : A) * F.C, tid % NT);
   constexpr int KP = (LC + 2 * NT - 1) / (2 * NT);
   constexpr bool kFull = LC % (2 * NT) == 0;
   double2 dA[KP], dB[KP];
@@ -438,7 +462,7 @@ __global__ __launch_bounds__(2 * fft_threads<LC>()) void k_fft_rows(FftArgs F, c
     dB[q] = Dp[B * LC + k2];
     wB[q] = wp[B * LC + k2];
   }
-  fft_first_global<LC, NT>(Yc + (size_t)(half ? B : A) * F.C, s + half * RSD, tid % NT, F.twC);
+  fft_first<LC, NT>(points, s + half * RSD, tid % NT, F.twC);
   const double2 *sA = s, *sB = s + RSD;
   double2 *hw = hw_out ? hw_out + (size_t)ch * (F.M + 1) : nullptr;
   double dh = 0.0, hh = 0.0;
@@ -509,6 +533,160 @@ __global__ __launch_bounds__(2 * fft_threads<LC>()) void k_fft_rows(FftArgs F, c
       partials[2 * q] = a;
       partials[2 * q + 1] = b;
     }
+  }
+}
+
+// ------------------------------------------- data and weights in bin order
+// H_k from Z_k and Z_(M-k) (E + W O, W = W_N^k), weighted, and its two sums.
+__device__ __forceinline__ void add_bin(double2 W, double2 zk, double2 zm, double2 d, double w, double &dh,
+                                        double &hh) {
+  const double2 E = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+  const double2 O = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+  const double2 WO = cmul(W, O);
+  const double2 x = make_double2((E.x + WO.x) * w, (E.y + WO.y) * w);
+  dh += x.x * d.x + x.y * d.y;
+  hh += x.x * x.x + x.y * x.y;
+}
+// Bins 0 and M, both real: H_0 = E_0 + O_0, H_M = E_0 - O_0.
+__device__ __forceinline__ void add_ends(double2 z0, double2 d0, double w0, double2 dm, double wm, double &dh,
+                                         double &hh) {
+  const double x0 = (z0.x + z0.y) * w0, xm = (z0.x - z0.y) * wm;
+  dh += x0 * d0.x + xm * dm.x;
+  hh += x0 * x0 + xm * xm;
+}
+
+// The workgroup's sums; valid in thread 0.
+template <int THREADS>
+__device__ __forceinline__ void block_sums(double &dh, double &hh) {
+  __shared__ double s_red[THREADS / 64][2];
+  for (int o = 32; o > 0; o >>= 1) {
+    dh += __shfl_xor(dh, o, 64);
+    hh += __shfl_xor(hh, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_red[threadIdx.x >> 6][0] = dh;
+    s_red[threadIdx.x >> 6][1] = hh;
+  }
+  __syncthreads();
+  dh = hh = 0.0;
+  for (int w = 0; w < THREADS / 64; w++) {
+    dh += s_red[w][0];
+    hh += s_red[w][1];
+  }
+}
+
+// Pass 2 for data and weights that a caller holds in bin order, k = k1 + R k2:
+// four neighbouring row pairs per workgroup, so that a step in k2 reads 64
+// bytes of data and 32 of weights per row group; the two workgroups that share
+// a 128-byte line run on one XCD.  Reading them so costs less than bringing
+// them into the row order first: 32 us at N = 2^21 where the row-ordered pass
+// takes 21 and the two transposes before it took 24.
+constexpr int kNatRows = 4;
+template <int LC>
+__global__ __launch_bounds__(2 * kNatRows * fft_threads<LC>()) void k_fft_rows_natural(FftArgs F, const double2 *Y,
+                                                                                       double *partials) {
+  constexpr int G = kNatRows, NT = fft_threads<LC>(), BS = 2 * G * NT, RSD = LC + LC / 16 + 1;
+  __shared__ double2 s[2 * G * RSD];
+  int ch, grp;
+  col_group<G>(ch, grp);
+  const int tid = threadIdx.x, r = tid % G, blk = grp * G + r;
+  const int A = blk, B = blk == 0 ? F.R / 2 : F.R - blk;
+  const double2 *Dp = F.Dp[ch];
+  const double *wp = F.wp[ch];
+  // the row of the wave's FFT (A rows first, then B rows), requested before the
+  // data: loads return in order, and the FFT waits for its points only
+  const int row = tid / NT, rb = grp * G + row % G;
+  const int k1 = row < G ? rb : (rb == 0 ? F.R / 2 : F.R - rb);
+  FirstPoints<LC, NT> points;
+  points.load(Y + (size_t)ch * F.M + (size_t)k1 * F.C, tid % NT);
+  // this thread's data and weights: rows A and B at k2 = (tid + q BS) / G
+  constexpr int KP = (G * LC + BS - 1) / BS;
+  constexpr bool kFull = G * LC % BS == 0;
+  double2 dA[KP], dB[KP];
+  double wA[KP], wB[KP];
+#pragma unroll
+  for (int q = 0; q < KP; q++) {
+    const int k2 = min((tid + q * BS) / G, LC - 1);
+    dA[q] = Dp[A + F.R * k2];
+    wA[q] = wp[A + F.R * k2];
+    dB[q] = Dp[B + F.R * k2];
+    wB[q] = wp[B + F.R * k2];
+  }
+  fft_first<LC, NT>(points, s + row * RSD, tid % NT, F.twC);
+  const double2 *sA = s + r * RSD, *sB = s + (G + r) * RSD;
+  const double2 WrA = tw2(F.twNhi, F.twNlo, A), WrB = tw2(F.twNhi, F.twNlo, B);
+  double dh = 0.0, hh = 0.0;
+#pragma unroll
+  for (int q = 0; q < KP; q++) {
+    const int k2 = (tid + q * BS) / G;
+    if (kFull || k2 < LC) {
+      const double2 t = F.twNr[k2];
+      if (blk == 0) {
+        if (k2 == 0) add_ends(sA[0], dA[q], wA[q], Dp[F.M], wp[F.M], dh, hh);
+        else add_bin(t, sA[pad(k2)], sA[pad(LC - k2)], dA[q], wA[q], dh, hh);
+        add_bin(cmul(WrB, t), sB[pad(k2)], sB[pad(LC - 1 - k2)], dB[q], wB[q], dh, hh);
+      } else {
+        add_bin(cmul(WrA, t), sA[pad(k2)], sB[pad(LC - 1 - k2)], dA[q], wA[q], dh, hh);
+        add_bin(cmul(WrB, t), sB[pad(k2)], sA[pad(LC - 1 - k2)], dB[q], wB[q], dh, hh);
+      }
+    }
+  }
+  block_sums<BS>(dh, hh);
+  if (tid == 0) {
+    const int q = ch * (F.R / (2 * G)) + grp;
+    partials[2 * q] = dh;
+    partials[2 * q + 1] = hh;
+  }
+}
+
+// Short series (M <= 4096): the whole inner product in one workgroup and one
+// launch, half of the threads per channel (R = 1, C = M; data and weights in
+// bin order).  Bound by latency: 9 us at N = 4096 (10 with the launch), where
+// five launches of the general form took 22.
+template <int M>
+__global__ __launch_bounds__(2 * fft_threads<M>()) void k_fft_small(FftArgs F, const double *h0, const double *h1,
+                                                                    double *out) {
+  constexpr int NT = fft_threads<M>(), RSD = M + M / 16, KP = (M / 2 + NT - 1) / NT;
+  __shared__ double2 s[2 * RSD];
+  const int ch = threadIdx.x / NT, t = threadIdx.x % NT;
+  const double2 *Dp = F.Dp[ch];
+  const double *wp = F.wp[ch];
+  FirstPoints<M, NT> points;
+  points.load(reinterpret_cast<const double2 *>(ch ? h1 : h0), t);
+  // bins k and M - k of this thread, k = t + q NT < M / 2
+  double2 dk[KP], dm[KP];
+  double wk[KP], wm[KP];
+#pragma unroll
+  for (int q = 0; q < KP; q++) {
+    const int k = min(t + q * NT, M / 2 - 1);
+    dk[q] = Dp[k];
+    wk[q] = wp[k];
+    dm[q] = Dp[M - k];
+    wm[q] = wp[M - k];
+  }
+  const double2 dc = Dp[M / 2];
+  const double wc = wp[M / 2];
+  double2 *x = s + ch * RSD;
+  fft_first<M, NT>(points, x, t, F.twC);
+  double dh = 0.0, hh = 0.0;
+#pragma unroll
+  for (int q = 0; q < KP; q++) {
+    const int k = t + q * NT;
+    if (k < M / 2) {
+      if (k == 0) {
+        add_ends(x[0], dk[q], wk[q], dm[q], wm[q], dh, hh);
+        add_bin(tw2(F.twNhi, F.twNlo, M / 2), x[pad(M / 2)], x[pad(M / 2)], dc, wc, dh, hh);
+      } else {
+        const double2 zk = x[pad(k)], zm = x[pad(M - k)];
+        add_bin(tw2(F.twNhi, F.twNlo, k), zk, zm, dk[q], wk[q], dh, hh);
+        add_bin(tw2(F.twNhi, F.twNlo, M - k), zm, zk, dm[q], wm[q], dh, hh);
+      }
+    }
+  }
+  block_sums<2 * NT>(dh, hh);
+  if (threadIdx.x == 0) {
+    out[0] = 4.0 * dh;
+    out[1] = 4.0 * hh;
   }
 }
 
@@ -831,6 +1009,42 @@ void launch_fft_final_reset(double *partials, int npairs, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- other lengths
+template <int LC>
+static void launch_natural(const FftArgs &F, const double2 *Y, double *partials, hipStream_t s) {
+  hipLaunchKernelGGL(k_fft_rows_natural<LC>, dim3(F.R / (2 * kNatRows), 2), dim3(2 * kNatRows * fft_threads<LC>()), 0,
+                     s, F, Y, partials);
+}
+
+int fft_natural_partials(const FftArgs &F) { return F.R / kNatRows; }
+
+void launch_fft_pass2_natural(const FftArgs &F, const double2 *Y, double *partials, hipStream_t s) {
+  switch (F.C) {
+    case 64: launch_natural<64>(F, Y, partials, s); break;
+    case 128: launch_natural<128>(F, Y, partials, s); break;
+    case 256: launch_natural<256>(F, Y, partials, s); break;
+    case 512: launch_natural<512>(F, Y, partials, s); break;
+    default: launch_natural<1024>(F, Y, partials, s); break;
+  }
+}
+
+template <int M>
+static void launch_small(const FftArgs &F, const double *h0, const double *h1, double *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_fft_small<M>, dim3(1), dim3(2 * fft_threads<M>()), 0, s, F, h0, h1, out);
+}
+
+bool launch_fft_small(const FftArgs &F, const double *h0, const double *h1, double *out, hipStream_t s) {
+  switch (F.M) {
+    case 128: launch_small<128>(F, h0, h1, out, s); break;
+    case 256: launch_small<256>(F, h0, h1, out, s); break;
+    case 512: launch_small<512>(F, h0, h1, out, s); break;
+    case 1024: launch_small<1024>(F, h0, h1, out, s); break;
+    case 2048: launch_small<2048>(F, h0, h1, out, s); break;
+    case 4096: launch_small<4096>(F, h0, h1, out, s); break;
+    default: return false;
+  }
+  return true;
+}
+
 // Columns of 2^a points, rows of 2^a, 3 2^a or 9 2^a.
 static const int kChirpRows[] = {16,  32,  48,  64,  96,  128, 144,  192,  256, 288,
                                  384, 512, 576, 768, 1024, 1152, 1536, 2048, 2304};

@@ -53,6 +53,14 @@ constexpr long long kFinalEmpty = 0x7FF4A5A5A5A5A5B1LL;  // a signalling NaN: no
 void launch_fft_pass2_final(const FftArgs &F, const double2 *Y, double *partials, const FftFinal &fin, hipStream_t s);
 void launch_fft_final_reset(double *partials, int npairs, hipStream_t s);
 
+// Data and weights in bin order (Dp, wp of M + 1 bins each).  Pass 2 for C from
+// 64 to 1024: fft_natural_partials(F) pairs.
+int fft_natural_partials(const FftArgs &F);
+void launch_fft_pass2_natural(const FftArgs &F, const double2 *Y, double *partials, hipStream_t s);
+// The whole inner product of a short series, M from 128 to 4096 with R = 1 and
+// C = M: out[0..1] = 4 x the sums.  False: another M.
+bool launch_fft_small(const FftArgs &F, const double *h0, const double *h1, double *out, hipStream_t s);
+
 // Lengths N = 2M whose half has a prime factor above 13: the M-point transform as a cyclic
 // convolution of length L = R C >= 2M - 1 (Bluestein), R from 2^a, C from 2^a,
 // 3 2^a and 9 2^a.

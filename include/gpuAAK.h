@@ -261,7 +261,7 @@ int aak_kerr_constants(double p, double e, double iota, double a, double *ELQ);
  * (re, im) doubles; ASDinv1/2: their weights; like_out: 2 doubles,
  * {4 <h w, d w>, 4 <h w, h w>} as aak_likelihood; stream: a hipStream_t or
  * NULL.  Limits: length a power of two in [2^8, 2^21] (else -2); scratch is
- * one static device array of about 80 MiB per GPU, held until the process
+ * one static device array of about 32 MiB per GPU, held until the process
  * ends; the first call at a new length copies that length's FFT tables and
  * waits for the copy, later calls only enqueue kernels; calls that overlap
  * on one GPU share the scratch and race.  Series and spectra 16-byte
