@@ -526,6 +526,7 @@ struct aak_mlp_s {
   float *X = nullptr, *T = nullptr, *loss = nullptr, *part = nullptr;
   int *idx = nullptr;
   int data_n = 0;
+  float *pin = nullptr;  // pinned: X | T of up to kPinRows rows, gradient, loss partials
   // inference scratch
   std::mutex mu;
   int icap = 0;
@@ -545,6 +546,12 @@ static void free_scratch(aak_mlp_s *m) {
   m->cap = 0;
   m->data_n = 0;
 }
+
+// Rows up to which a gradient call passes its data through pinned memory, read
+// and written by the kernels themselves: 56 us a call at 4096 rows against 90
+// with two uploads and two downloads, 46 against 121 at 64, 83 against 120 at
+// 16384.  Longer calls upload, so the buffer stays at 0.6 MB.
+constexpr int kPinRows = 16384;
 
 static int grad_groups(int B) { return std::min(kGradGroups, (B + GROWS - 1) / GROWS); }
 
@@ -573,17 +580,23 @@ static int grow_scratch(aak_mlp_s *m, int B, int data) {
   return 0;
 }
 
-// One forward + backward over rows idx[0 .. B) of the uploaded data (idx null:
-// its first B);
-// with step > 0 an Adam update.  loss_sum (optional) gets the squared error.
-static int train_step(aak_mlp_s *m, const int *idx, int B, float lr, bool update, double *loss_sum) {
+// One forward + backward over rows idx[0 .. B) of X, T (idx null: the first B);
+// with `update` an Adam step.
+static void launch_step(aak_mlp_s *m, const float *X, const float *T, const int *idx, int B, float lr, bool update,
+                        float *grad, float *loss) {
   const int groups = grad_groups(B);
   const float dscale = 2.f / (3.f * (float)B);
-  hipLaunchKernelGGL(k_mlp_gradient, dim3(groups), dim3(kGradThreads), 0, m->s, m->X, m->T, idx, B, m->P, m->Pb, m->Wt,
-                     m->part, m->loss, dscale);
+  hipLaunchKernelGGL(k_mlp_gradient, dim3(groups), dim3(kGradThreads), 0, m->s, X, T, idx, B, m->P, m->Pb, m->Wt,
+                     m->part, loss, dscale);
   if (update) m->step++;
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kNP + 63) / 64), dim3(kThreads), 0, m->s, groups, m->part, m->grad, m->P, m->Pb,
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kNP + 63) / 64), dim3(kThreads), 0, m->s, groups, m->part, grad, m->P, m->Pb,
                      m->Wt, m->m1, m->m2, update ? m->step : 0, lr, 0.9f, 0.999f, 1e-8f);
+}
+
+// launch_step over the uploaded data.  loss_sum (optional) gets the squared error.
+static int train_step(aak_mlp_s *m, const int *idx, int B, float lr, bool update, double *loss_sum) {
+  const int groups = grad_groups(B);
+  launch_step(m, m->X, m->T, idx, B, lr, update, m->grad, m->loss);
   MLPCHK(hipGetLastError());
   if (loss_sum) {
     std::vector<float> lp(groups);
@@ -695,6 +708,7 @@ int aak_mlp_destroy(aak_mlp m) {
   if (!m) return fail(-1, "null model");
   if (m->s) (void)hipStreamSynchronize(m->s);
   free_scratch(m);
+  if (m->pin) (void)hipHostFree(m->pin);
   void *ps[] = {m->P, m->m1, m->m2, m->grad, m->Pb, m->Wt, m->iX, m->iY};
   for (void *p : ps)
     if (p) (void)hipFree(p);
@@ -750,6 +764,26 @@ int aak_mlp_forward(aak_mlp m, const float *X, int n, float *Y) {
 int aak_mlp_gradient(aak_mlp m, const float *X, const float *T, int n, float *grad, double *loss) {
   if (!m || !X || !T || !grad || n <= 0) return fail(-2, "bad argument");
   MLPCHK(hipSetDevice(m->dev));
+  if (n <= kPinRows) {
+    // the kernels read the rows from pinned host memory, each once, and leave
+    // the gradient there
+    int rc = grow_scratch(m, n, 0);
+    if (rc) return rc;
+    if (!m->pin)
+      MLPCHK(hipHostMalloc((void **)&m->pin, sizeof(float) * (7 * (size_t)kPinRows + kNP + kGradGroups),
+                           hipHostMallocDefault));
+    float *pX = m->pin, *pT = pX + 4 * (size_t)kPinRows, *pG = pT + 3 * (size_t)kPinRows, *pL = pG + kNP;
+    std::memcpy(pX, X, sizeof(float) * 4 * (size_t)n);
+    std::memcpy(pT, T, sizeof(float) * 3 * (size_t)n);
+    launch_step(m, pX, pT, nullptr, n, 0.f, false, pG, pL);
+    MLPCHK(hipGetLastError());
+    MLPCHK(hipStreamSynchronize(m->s));
+    std::memcpy(grad, pG, sizeof(float) * kNP);
+    double ls = 0.0;
+    for (int g = 0; g < grad_groups(n); g++) ls += pL[g];
+    if (loss) *loss = ls / (3.0 * n);
+    return 0;
+  }
   int rc = grow_scratch(m, n, n);
   if (rc) return rc;
   MLPCHK(hipMemcpyAsync(m->X, X, sizeof(float) * 4 * (size_t)n, hipMemcpyHostToDevice, m->s));
