@@ -35,7 +35,7 @@ namespace aak {
 // ------------------------------------------------------------------ rates
 constexpr int kRatesThreads = kRatesBlock;
 constexpr int kRatesSlots = 1024;  // workgroups that run at once: 4 per CU
-constexpr int kStageCap = 128;  // knot intervals staged in LDS per block (else direct evaluation)
+constexpr int kStageCap = 256;  // knot intervals staged in LDS per block (else direct evaluation)
 
 __device__ inline int knot_search(const double *x, int lo, int hi, double t) {
   // largest k in [lo, hi-1] with x[k] <= t (hi is exclusive upper knot)
@@ -255,7 +255,13 @@ __global__ __launch_bounds__(kRatesThreads, 4) void k_rates(DenseParams P, Dense
 
 void launch_rates(const DenseParams &P, const DenseBuffers &B, hipStream_t s) {
   const long long last = rates_last(P), slots = (long long)kRatesThreads * kRatesSlots;
-  const int per = (int)std::max(1LL, (last + slots - 1) / slots);
+  // no more samples than LDS holds knots for (fast sources have a knot every few
+  // samples, beyond it every sample searches the table): with a knot per 10
+  // samples the stage takes 50 us at N = 2^21, 72 without this limit (60 with
+  // one sample per thread); with one per 3.5 samples 51, 71 (56)
+  const double rows = (kStageCap - 8) * P.grid.dt_large / (kRatesThreads * P.dt);
+  const int most = rows < 1.0 ? 1 : rows < 64.0 ? (int)rows : 64;
+  const int per = (int)std::min((long long)most, std::max(1LL, (last + slots - 1) / slots));
   const int nb = (int)std::max(1LL, (last + kRatesThreads * per - 1) / (kRatesThreads * per));
   hipLaunchKernelGGL(k_rates, dim3(nb), dim3(kRatesThreads), 0, s, P, B, per);
 }
