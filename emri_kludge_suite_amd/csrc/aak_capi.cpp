@@ -207,7 +207,6 @@ struct Lane {
   int *d_ms_p = nullptr;
   int *d_ms_slot = nullptr;
   int *d_ms_list = nullptr;
-  int *d_ms_split = nullptr;
   double *d_ms_eref = nullptr;
   rocfft_plan plan = nullptr;
   rocfft_execution_info exec = nullptr;
@@ -315,7 +314,6 @@ struct aak_handle_s {
     B.ms_p = ln.d_ms_p;
     B.ms_slot = ln.d_ms_slot;
     B.ms_list = ln.d_ms_list;
-    B.ms_split = ln.d_ms_split;
     B.ms_eref = ln.d_ms_eref;
     B.bessel_c = d_bessel;
     B.bessel_lgf = d_bessel + (size_t)(kBesselKMax + 1) * kBesselMMax;
@@ -340,7 +338,6 @@ static int alloc_lane(aak_handle h, Lane &L) {
   HIPCHK(hipMalloc(&L.d_ms_p, sizeof(int) * ((size_t)N / 256 + 4)));
   HIPCHK(hipMalloc(&L.d_ms_slot, sizeof(int) * ((size_t)N / 256 + 4)));
   HIPCHK(hipMalloc(&L.d_ms_list, sizeof(int) * ((size_t)N / 256 + 4)));
-  HIPCHK(hipMalloc(&L.d_ms_split, sizeof(int) * ((size_t)N / 256 + 4)));
   HIPCHK(hipMalloc(&L.d_ms_eref, sizeof(double) * 2 * ((size_t)N / 256 + 4)));
   const int nblk = (N + kFoldBlock - 1) / kFoldBlock + 1;
   L.fold_nblk_cap = nblk;
@@ -436,7 +433,7 @@ static void free_lane(Lane &L) {
   if (L.exec) rocfft_execution_info_destroy(L.exec);
   void *ptrs[] = {L.d_table[0], L.d_table[1], L.d_dense, L.d_h, L.d_t, L.d_flags, L.d_guardw, L.d_foldmem,
                   L.d_hf, L.d_fy, L.d_fz, L.d_partials, L.d_fparts, L.d_like, L.d_work, L.d_ms_coef, L.d_ms_p, L.d_ms_slot,
-                  L.d_ms_list, L.d_ms_split, L.d_ms_eref};
+                  L.d_ms_list, L.d_ms_eref};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (int k = 0; k < 2; k++) {

@@ -210,7 +210,6 @@ struct DenseBuffers {
   int *ms_p;                       // [256-sample blocks] Taylor order (-1: per-sample path)
   int *ms_slot;                    // [256-sample blocks] coefficient slot of the block's expansion
   int *ms_list;                    // [256-sample blocks] blocks of the per-sample path (count in flags[2])
-  int *ms_split;                   // [expansion blocks] blocks expanded again per 256 samples (count in flags[4])
   double *ms_eref;                 // [slots] expansion point
   const double *bessel_c;          // series coefficients c_m(k)
   const double *bessel_lgf;        // log(k!)

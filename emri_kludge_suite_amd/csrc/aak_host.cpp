@@ -851,11 +851,13 @@ int plan_waveform(const WaveConfig &cfg, const SourceParams &sp, WaveformPlan *p
   P.bessel_series = (nmodes <= kMaxModes && e_bound <= kSeriesMaxE) ? 1 : 0;
   P.e_series = P.bessel_series ? e_bound : 0.0;
   P.mixed = cfg.mixed ? 1 : 0;
-  // FP64: one expansion per 1024 samples from the length on where each CU still
-  // gets one (2^18); setup and sum together, 256 against 1024 samples per
+  // FP64: one expansion per 1024 samples from the signal length on where each CU
+  // still gets one (2^18); setup and sum together, 256 against 1024 samples per
   // expansion: N = 2^21 228 against 190 us, 2^18 37.4 against 34.3, but 2^16
-  // 21.1 against 24.0 and 2^15 30 against 35 (one wave works on each expansion)
-  P.xshift = cfg.exp_shift >= 0 ? cfg.exp_shift : (cfg.mixed || N >= (1 << 18) ? 2 : 0);
+  // 21.1 against 24.0, 2^15 30 against 35 (one wave works on each expansion), and
+  // 127 against 141 for a source that plunges at sample 46421 of 2^18
+  const int signal = std::min(N, P.ip + P.ib);
+  P.xshift = cfg.exp_shift >= 0 ? cfg.exp_shift : (cfg.mixed || signal >= (1 << 18) ? 2 : 0);
   P.full_dense = 1;
   {
     // mixed form: E1 = sin(lam) S - cos(lam) (cos a e1 + sin a e2) and

@@ -22,7 +22,7 @@ struct WaveConfig {
   int n_max = 0;  // > 0 overrides the reference harmonic rule
   int mixed = 0;  // 1: mixed-precision mode sum
   // mode-sum expansion blocks of 256 << exp_shift samples; -1: 2 in the
-  // mixed form and in FP64 from 2^18 samples on, else 0 (any value keeps the
+  // mixed form and in FP64 from 2^18 signal samples on, else 0 (any value keeps the
   // accuracy: the Taylor order adapts, blocks beyond order 8 are expanded per
   // 256 samples, and what is beyond it then takes the per-sample path)
   int exp_shift = -1;

@@ -2237,7 +2237,7 @@ __device__ inline double harmonic_phase(const DenseParams &P, const SampleGeom &
 constexpr int kMsThreads = 256;
 constexpr int kTaylorModes = 128;
 // Samples per expansion block: 256 << exp_shift (host-set, default 2 in the
-// mixed form and in FP64 from 2^18 samples on, else 0).  One expansion serves
+// mixed form and in FP64 from 2^18 signal samples on, else 0).  One expansion serves
 // 1024 samples while the setup work falls fourfold and the mean order rises
 // little (mixed, over the production prior: from 2.0 to 2.5); blocks that need
 // more than order 8 are expanded per 256 samples.
@@ -2324,91 +2324,77 @@ __device__ inline void setup_slot(const DenseParams &P, const DenseBuffers &B, i
   }
 }
 
-// Block setup, one wave per expansion block of 256 << xs samples: the range
-// of e over the block's signal samples, the order p and e_ref (every lane
-// derives the same values from a butterfly reduction), then one harmonic per
-// lane.  The Bessel run of a lane is staged in LDS (dynamic orders) and the
+// Block setup, 2^xs waves per expansion block of 256 << xs samples, the first
+// waves of all blocks before the second ones.  Each finds the range of e over
+// the block's signal samples, the order p and e_ref (every lane derives the same
+// values from a butterfly reduction); the first wave then expands, one harmonic
+// per lane.  The Bessel run of a lane is staged in LDS (dynamic orders) and the
 // expansion is formed in registers.  An expansion block of more than 256
 // samples that no order up to kTaylorMax serves (fast evolution near a
-// plunge) is listed for k_modesum_split (count in flags[4]); other failures
-// (no Bessel series: e > kSeriesMaxE, more than kTaylorModes harmonics) list
-// the block's 256-sample blocks for the per-sample path.  A block with no
-// signal sample gets p = 0 and no coefficients.
+// plunge) is expanded per 256 samples (slot ne + blk; flags[4] counts such
+// blocks), one by each of its waves, which otherwise end with their look at the
+// range: 3 us a waveform at N = 2^21, where a launch behind the setup that walked
+// a list of such blocks took 5 with an empty list and 12 to 18 more with 14 to
+// 58 of them (setup and sum in FP64 127 and 198 against 115 and 182 us).
+// Other failures (no Bessel series: e > kSeriesMaxE, more than kTaylorModes
+// harmonics; 256 samples beyond order kTaylorMax) list the 256-sample blocks for
+// the per-sample path.  A block with no signal sample gets p = 0 and no
+// coefficients.
 template <bool MIXED>
 __global__ __launch_bounds__(kSetupThreads) void k_modesum_setup(DenseParams P, DenseBuffers B, FoldArgs FA,
                                                                  FoldWork FW, int ne) {
   __shared__ double s_J[kTaylorOrders][kSetupThreads];
-  const int lane = threadIdx.x, eb = blockIdx.x;
-  if (eb >= ne) {
-    // workgroups past the expansion blocks: the serial replay of a phase
+  const int xs = exp_shift(P), span = kMsThreads << xs, sub = 1 << xs;
+  const int lane = threadIdx.x, part = blockIdx.x / ne, eb = blockIdx.x % ne;
+  if (part >= sub) {
+    // workgroups past the expansion blocks': the serial replay of a phase
     // whose single-pass fold failed (the setup reads e only)
-    const int p = eb - ne;
+    const int p = blockIdx.x - ne * sub;
     if (FW.status[p]) fold_serial_replay(FA, FW, p, &s_J[0][0], kTaylorOrders * kSetupThreads);
     return;
   }
   const int n_end = min(P.N, P.ip + P.ib);
-  const int xs = exp_shift(P), span = kMsThreads << xs, sub = 1 << xs;
   const int nb = (P.N + 2 + kMsThreads - 1) / kMsThreads;
   double lo, hi;
   e_range(B, eb * span, span, n_end, lo, hi);
-  const bool any = lo <= hi;
+  const double tol = MIXED ? kTaylorTolFp32 : kTaylorTolFp64;
+  bool any = lo <= hi;
   const bool series = P.bessel_series && P.nmodes <= kTaylorModes && hi <= P.e_series;
-  int p = -1;
+  int p = -1, slot = eb, first = eb * sub, end = min(nb, first + sub);
   double eref = 0.0;
   if (!any) {
     p = 0;
   } else if (series) {
     eref = 0.5 * (lo + hi);
-    p = taylor_order(P.nmodes, 0.5 * (hi - lo), MIXED ? kTaylorTolFp32 : kTaylorTolFp64);
+    p = taylor_order(P.nmodes, 0.5 * (hi - lo), tol);
   }
-  const bool split = p < 0 && series && sub > 1;
+  if (p < 0 && series && sub > 1) {
+    if (part == 0 && lane == 0) atomicAdd(&B.flags[4], 1);
+    first += part;
+    if (first >= nb) return;
+    end = first + 1;
+    slot = ne + first;
+    e_range(B, first * kMsThreads, kMsThreads, n_end, lo, hi);
+    any = lo <= hi;
+    p = 0;
+    eref = 0.0;
+    if (any) {
+      eref = 0.5 * (lo + hi);
+      p = taylor_order(P.nmodes, 0.5 * (hi - lo), tol);
+    }
+  } else if (part > 0) {
+    return;
+  }
   if (lane == 0) {
-    B.ms_eref[eb] = eref;
-    if (split) B.ms_split[atomicAdd(&B.flags[4], 1)] = eb;
-    for (int blk = eb * sub; blk < min(nb, eb * sub + sub); blk++) {
+    B.ms_eref[slot] = eref;
+    for (int blk = first; blk < end; blk++) {
       B.ms_p[blk] = p;
-      B.ms_slot[blk] = eb;
-      if (p < 0 && !split) B.ms_list[atomicAdd(&B.flags[2], 1)] = blk;
+      B.ms_slot[blk] = slot;
+      if (p < 0) B.ms_list[atomicAdd(&B.flags[2], 1)] = blk;
     }
   }
   if (p < 0 || !any) return;
-  setup_slot<MIXED>(P, B, eb, p, eref, &s_J[0][lane]);
-}
-
-// The 256-sample blocks of the expansion blocks listed by k_modesum_setup,
-// each expanded on its own (slot ne + blk), one wave per block over a fixed
-// grid; blocks that still need an order above kTaylorMax go to the
-// per-sample path.  Returns at once when nothing was listed.
-constexpr int kSplitGrid = 256;
-template <bool MIXED>
-__global__ __launch_bounds__(kSetupThreads) void k_modesum_split(DenseParams P, DenseBuffers B, int ne) {
-  const int count = B.flags[4];
-  if (count == 0) return;
-  __shared__ double s_J[kTaylorOrders][kSetupThreads];
-  const int lane = threadIdx.x, sub = 1 << exp_shift(P);
-  const int n_end = min(P.N, P.ip + P.ib);
-  const int nb = (P.N + 2 + kMsThreads - 1) / kMsThreads;
-  for (int k = blockIdx.x; k < count * sub; k += gridDim.x) {
-    const int blk = B.ms_split[k / sub] * sub + k % sub;
-    if (blk >= nb) continue;
-    double lo, hi;
-    e_range(B, blk * kMsThreads, kMsThreads, n_end, lo, hi);
-    const bool any = lo <= hi;
-    int p = 0;
-    double eref = 0.0;
-    if (any) {
-      eref = 0.5 * (lo + hi);
-      p = taylor_order(P.nmodes, 0.5 * (hi - lo), MIXED ? kTaylorTolFp32 : kTaylorTolFp64);
-    }
-    const int slot = ne + blk;
-    if (lane == 0) {
-      B.ms_p[blk] = p;
-      B.ms_slot[blk] = slot;
-      B.ms_eref[slot] = eref;
-      if (p < 0) B.ms_list[atomicAdd(&B.flags[2], 1)] = blk;
-    }
-    if (p >= 0 && any) setup_slot<MIXED>(P, B, slot, p, eref, &s_J[0][lane]);
-  }
+  setup_slot<MIXED>(P, B, slot, p, eref, &s_J[0][lane]);
 }
 
 int modesum_blocks(const DenseParams &P) { return (P.N + 2 + kMsThreads - 1) / kMsThreads; }
@@ -2706,15 +2692,12 @@ void launch_modesum(const DenseParams &P, const DenseBuffers &B, const FoldArgs 
   const int nb = modesum_blocks(P), ne = expansion_blocks(P);
   const FoldArgs FA = replay ? *replay : FoldArgs{};
   const FoldWork FW = fw ? *fw : FoldWork{};
-  const int ng = ne + (replay ? 3 : 0);
+  const int ng = (ne << exp_shift(P)) + (replay ? 3 : 0);
   if (P.mixed) {
     hipLaunchKernelGGL(k_modesum_setup<true>, dim3(ng), dim3(kSetupThreads), 0, s, P, B, FA, FW, ne);
-    if (exp_shift(P) > 0) hipLaunchKernelGGL(k_modesum_split<true>, dim3(kSplitGrid), dim3(kSetupThreads), 0, s, P, B, ne);
     hipLaunchKernelGGL(k_modesum<true>, dim3(nb), dim3(kMsThreads), 0, s, P, B, nb);
   } else {
     hipLaunchKernelGGL(k_modesum_setup<false>, dim3(ng), dim3(kSetupThreads), 0, s, P, B, FA, FW, ne);
-    if (exp_shift(P) > 0)
-      hipLaunchKernelGGL(k_modesum_split<false>, dim3(kSplitGrid), dim3(kSetupThreads), 0, s, P, B, ne);
     hipLaunchKernelGGL(k_modesum<false>, dim3(nb), dim3(kMsThreads), 0, s, P, B, nb);
   }
   hipLaunchKernelGGL(k_modesum_direct, dim3(kDirectGrid), dim3(kMsThreads), 0, s, P, B);

@@ -99,7 +99,7 @@ int aak_get_pool_stats(aak_handle h, double *out, int n);
  * not depend on it beyond the mixed form's FP32 rounding): feed_depth = short
  * host plans kept ready for the GPU (1..256; < 0 keeps it), expansion_shift =
  * mode-sum expansion blocks of 256 << shift samples (0..3; -1 keeps it, -2
- * restores the default: 2 mixed and FP64 from 2^18 samples on, else 0). */
+ * restores the default: 2 mixed and FP64 from 2^18 signal samples on, else 0). */
 int aak_set_tuning(aak_handle h, int feed_depth, int expansion_shift);
 
 /* Concurrent streams ("lanes", 1..8) over which aak_likelihood_batch spreads
