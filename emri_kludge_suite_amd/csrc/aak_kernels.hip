@@ -2333,9 +2333,9 @@ __device__ inline void setup_slot(const DenseParams &P, const DenseBuffers &B, i
 // samples that no order up to kTaylorMax serves (fast evolution near a
 // plunge) is expanded per 256 samples (slot ne + blk; flags[4] counts such
 // blocks), one by each of its waves, which otherwise end with their look at the
-// range: 3 us a waveform at N = 2^21, where a launch behind the setup that walked
-// a list of such blocks took 5 with an empty list and 12 to 18 more with 14 to
-// 58 of them (setup and sum in FP64 127 and 198 against 115 and 182 us).
+// range.  A launch behind the setup that walked a list of such blocks took 5 us
+// with an empty list (setup and sum, mixed, N = 2^21: 101 against 98 us) and 12
+// to 18 more with 14 to 58 of them (FP64: 127 and 198 against 115 and 182).
 // Other failures (no Bessel series: e > kSeriesMaxE, more than kTaylorModes
 // harmonics; 256 samples beyond order kTaylorMax) list the 256-sample blocks for
 // the per-sample path.  A block with no signal sample gets p = 0 and no
@@ -2345,14 +2345,18 @@ __global__ __launch_bounds__(kSetupThreads) void k_modesum_setup(DenseParams P, 
                                                                  FoldWork FW, int ne) {
   __shared__ double s_J[kTaylorOrders][kSetupThreads];
   const int xs = exp_shift(P), span = kMsThreads << xs, sub = 1 << xs;
-  const int lane = threadIdx.x, part = blockIdx.x / ne, eb = blockIdx.x % ne;
+  // the waves of a block lie a multiple of 8 workgroups apart: one XCD, whose
+  // L2 then holds the block's e (17 against 66 MB read, 98 against 102 us)
+  const int stride = (ne + 7) & ~7;
+  const int lane = threadIdx.x, part = blockIdx.x / stride, eb = blockIdx.x % stride;
   if (part >= sub) {
     // workgroups past the expansion blocks': the serial replay of a phase
     // whose single-pass fold failed (the setup reads e only)
-    const int p = blockIdx.x - ne * sub;
+    const int p = blockIdx.x - stride * sub;
     if (FW.status[p]) fold_serial_replay(FA, FW, p, &s_J[0][0], kTaylorOrders * kSetupThreads);
     return;
   }
+  if (eb >= ne) return;
   const int n_end = min(P.N, P.ip + P.ib);
   const int nb = (P.N + 2 + kMsThreads - 1) / kMsThreads;
   double lo, hi;
@@ -2692,7 +2696,7 @@ void launch_modesum(const DenseParams &P, const DenseBuffers &B, const FoldArgs 
   const int nb = modesum_blocks(P), ne = expansion_blocks(P);
   const FoldArgs FA = replay ? *replay : FoldArgs{};
   const FoldWork FW = fw ? *fw : FoldWork{};
-  const int ng = (ne << exp_shift(P)) + (replay ? 3 : 0);
+  const int ng = (((ne + 7) & ~7) << exp_shift(P)) + (replay ? 3 : 0);
   if (P.mixed) {
     hipLaunchKernelGGL(k_modesum_setup<true>, dim3(ng), dim3(kSetupThreads), 0, s, P, B, FA, FW, ne);
     hipLaunchKernelGGL(k_modesum<true>, dim3(nb), dim3(kMsThreads), 0, s, P, B, nb);
