@@ -1671,6 +1671,31 @@ int aak_test_inspiral_rates(double p, double e, double cosi, double a, double *o
   return inspiral_rates<HostCx>(p, e, cosi, a, out);
 }
 
+int aak_test_circular_energies(const double *orbits, int n, double *E) {
+  if (n < 0 || (n > 0 && (!orbits || !E))) return fail(-2, "bad arguments");
+  CircularOrbit::Hint hint;
+  for (int k = 0; k < n; k++) {
+    const double *o = orbits + 3 * k;
+    CircularOrbit found, plain;
+    E[2 * k] = found.init(o[0], o[1], o[2], &hint) ? std::nan("") : found.E;
+    E[2 * k + 1] = plain.init(o[0], o[1], o[2], nullptr, true) ? std::nan("") : plain.E;
+  }
+  return n;
+}
+
+int aak_test_eccentric(double p, double e, double cosi, double a, double dt, int maxsteps, double *out) {
+  if (!out || maxsteps < 1 || maxsteps > 100) return fail(-2, "bad arguments");
+  Inspiral<HostCx> insp;
+  if (insp.init(a)) return fail(-1, "LSO table failed");
+  InspiralPoint pts[100];
+  const int n = insp.eccentric(p, e, cosi, dt, maxsteps, pts);
+  for (int k = 0; k < n; k++) {
+    const double q[4] = {pts[k].t, pts[k].p, pts[k].e, pts[k].cosi};
+    std::copy(q, q + 4, out + 4 * k);
+  }
+  return n;
+}
+
 int aak_test_inner_product(aak_handle h, const double *hI, const double *hII, double *like, double *spec,
                            int *fused) {
   if (!h) return fail(-1, "null handle");

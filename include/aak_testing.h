@@ -45,6 +45,16 @@ int aak_test_taylor_amplitudes(int n_max, int n, double e_ref, double del, doubl
 /* One evaluation of the inspiral rates (dp/dt, de/dt, dcos(iota)/dt). */
 int aak_test_inspiral_rates(double p, double e, double cosi, double a, double *out);
 
+/* Energies of n circular orbits, orbits[3k..] = (cos(iota), r, a), found one
+ * after another as the inspiral does: E[2k] with the root of the orbit before
+ * as a start, E[2k+1] by the plain bisection (NaN: no orbit).  Returns n. */
+int aak_test_circular_energies(const double *orbits, int n, double *E);
+
+/* The inspiral alone from (p, e, cos(iota)) at spin a in steps of dt (units of
+ * M^2/mu): out[4k..] = (t, p, e, cos(iota)) of up to maxsteps <= 100 points.
+ * Returns their number or < 0. */
+int aak_test_eccentric(double p, double e, double cosi, double a, double dt, int maxsteps, double *out);
+
 /* The inner-product stage alone on two given real series of length `length`
  * (the handle's data and weights from aak_input_data): like[0..1] =
  * (<h|d>, <h|h>) as aak_Likelihood returns them, spec (optional) =
