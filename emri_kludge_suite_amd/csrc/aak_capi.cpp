@@ -10,7 +10,7 @@
 //     one template's narrow kernels overlap another's wide ones,
 //   * the inner-product stage: for power-of-two lengths the fused four-step
 //     FFT + weighted reduction (aak_fft.hip, data stored in its row order),
-//     for lengths whose half has a prime factor above 13 the convolution of
+//     for lengths whose half has a prime factor above 17 the convolution of
 //     the same file, otherwise a rocFFT real-forward plan per lane (both
 //     channels in one batched call) and the separate reduction; the Bessel
 //     tables,
@@ -237,7 +237,7 @@ struct aak_handle_s {
   double2 *d_data = nullptr;      // [2][nbins] weighted data (fused FFT path: in its row order)
   double *d_w = nullptr;          // [2][nbins] weights (same order as d_data)
   bool fused_fft = false;         // power-of-two length: fused FFT + reduction
-  bool chirp_fft = false;         // N/2 with a prime factor above 13: Bluestein's convolution, else rocFFT
+  bool chirp_fft = false;         // N/2 with a prime factor above 17: Bluestein's convolution, else rocFFT
   FftArgs fft{};
   ChirpArgs chirp{};
   double2 *d_fft_tw = nullptr;    // twiddle tables of the fused FFT
@@ -442,6 +442,15 @@ static void free_lane(Lane &L) {
   }
   if (L.stream) (void)hipStreamDestroy(L.stream);
   L = Lane();
+}
+
+// Transform of the inner-product stage at a length, and its factors R x C.
+enum { kLibrary = 0, kFourStep = 1, kConvolution = 2 };
+static int transform_of(int length, int *R, int *C) {
+  // AAK_FFT=rocfft keeps the library transform for every length
+  const char *env = std::getenv("AAK_FFT");
+  if (env && std::strcmp(env, "rocfft") == 0) return kLibrary;
+  return fft_supported(length, R, C) ? kFourStep : chirp_supported(length, R, C) ? kConvolution : kLibrary;
 }
 
 static int alloc_handle(aak_handle h) {
@@ -898,17 +907,15 @@ int aak_create(double T_fit, int init_length, int length, double init_dt, double
     h->nlanes = v < 1 ? 1 : (v > kMaxLanes ? kMaxLanes : v);
   }
   {
-    // AAK_FFT=rocfft keeps the library transform for every length
-    const char *env = std::getenv("AAK_FFT");
-    const bool library = env && std::strcmp(env, "rocfft") == 0;
     int R = 0, C = 0;
-    if (!library && fft_supported(length, &R, &C)) {
+    const int form = transform_of(length, &R, &C);
+    if (form == kFourStep) {
       h->fused_fft = true;
       h->fft.N = length;
       h->fft.M = length / 2;
       h->fft.R = R;
       h->fft.C = C;
-    } else if (!library && chirp_supported(length, &R, &C)) {
+    } else if (form == kConvolution) {
       h->chirp_fft = true;
       h->chirp.N = length;
       h->chirp.M = length / 2;
@@ -1694,6 +1701,14 @@ int aak_test_eccentric(double p, double e, double cosi, double a, double dt, int
     std::copy(q, q + 4, out + 4 * k);
   }
   return n;
+}
+
+int aak_test_transform(int length, int *R, int *C) {
+  int r = 0, c = 0;
+  const int form = transform_of(length, &r, &c);
+  if (R) *R = form == kLibrary ? 0 : r;
+  if (C) *C = form == kLibrary ? 0 : c;
+  return form;
 }
 
 int aak_test_inner_product(aak_handle h, const double *hI, const double *hII, double *like, double *spec,

@@ -696,7 +696,8 @@ __global__ __launch_bounds__(2 * fft_threads<M>()) void k_fft_small(FftArgs F, c
 //   Z_k = c_k sum_m (z_m c_m) conj(c_(k-m)),
 // a cyclic convolution of length L >= 2M - 1 with a fixed filter, whose
 // transform F is formed once per handle.  L = R C with R from 2^a, C from 2^a,
-// 3 2^a and 9 2^a, at most a third longer than it must be from N = 512 on.
+// 3 2^a and 9 2^a, at most half longer than it must be from N = 514 on and a
+// third from 1538 on.
 // Both transforms of the convolution run in the four-step form above, and what
 // lies between them stays in LDS:
 //   k_chirp_cols   columns b of z_m c_m (zero from M on), times W_L^(b k1);
@@ -1049,16 +1050,19 @@ bool launch_fft_small(const FftArgs &F, const double *h0, const double *h1, doub
 static const int kChirpRows[] = {16,  32,  48,  64,  96,  128, 144,  192,  256, 288,
                                  384, 512, 576, 768, 1024, 1152, 1536, 2048, 2304};
 
-// Lengths whose half is a product of primes up to 13 stay with the library's
+// Lengths whose half is a product of primes up to 17 stay with the library's
 // mixed-radix transforms, which need no convolution for them: at N = 2000000 they
 // take 106 us against 183 of the convolution, at 250000 39 against 46, at 4000
-// 22 against 29.  For all others the library runs a convolution too, and this
-// one is faster throughout (N = 2103840: 196 us against 781, 1048578: 107
-// against 384, 65538: 37 against 56, 4002: 29 against 44, 1002: 23 against 30).
+// 22 against 29; with the factor 17 119 against 198 at N = 2228224, 131 against
+// 202 at 2263040, 41 against 53 at 278528, 28 against 32 at 8704.  With a factor
+// from 19 on the library runs a convolution too, and this one is faster (N =
+// 2490368 = 19 2^17: 242 us against 787, 2103840: 196 against 781, 1048578: 107
+// against 384, 65538: 37 against 56, 4002: 29 against 44, 1002: 23 against 30,
+// 74: 25 against 27) but for the shortest (38 to 62: 26 against 23).
 bool chirp_supported(int N, int *R, int *C) {
-  if (N < 16 || (N & 1)) return false;
+  if (N < 64 || (N & 1)) return false;
   int rest = N / 2;
-  for (int q : {2, 3, 5, 7, 11, 13})
+  for (int q : {2, 3, 5, 7, 11, 13, 17})
     while (rest % q == 0) rest /= q;
   if (rest == 1) return false;
   const long long need = (long long)N - 1;  // 2M - 1

@@ -61,7 +61,7 @@ void launch_fft_pass2_natural(const FftArgs &F, const double2 *Y, double *partia
 // C = M: out[0..1] = 4 x the sums.  False: another M.
 bool launch_fft_small(const FftArgs &F, const double *h0, const double *h1, double *out, hipStream_t s);
 
-// Lengths N = 2M whose half has a prime factor above 13: the M-point transform as a cyclic
+// Lengths N = 2M whose half has a prime factor above 17: the M-point transform as a cyclic
 // convolution of length L = R C >= 2M - 1 (Bluestein), R from 2^a, C from 2^a,
 // 3 2^a and 9 2^a.
 // Tables as in FftArgs (W_L in place of W_M); chirp: exp(-i pi m^2 / M), m < M;
@@ -70,8 +70,8 @@ struct ChirpArgs {
   int N, M, L, R, C;
   const double2 *twR, *twC, *twLlo, *twLhi, *twNlo, *twNhi, *chirp, *filter;
 };
-// Lengths handled (even, up to 4194304, N/2 with a prime factor above 13) and
-// the smallest R C for them.
+// Lengths handled (even, from 64 to 4718590, N/2 with a prime factor above 17)
+// and the smallest R C for them.
 bool chirp_supported(int N, int *R, int *C);
 int chirp_partials(const ChirpArgs &F);
 // Size of the tables (double2 entries); the part the host fills (its size, and

@@ -216,7 +216,7 @@ class GPUAAK:
         fft / dot: for power-of-two lengths the column pass of the fused FFT,
         then the row pass with the weighting and both sums; otherwise the
         transform (the library's own convolution where length/2 has a prime
-        factor above 13, else rocFFT), then the weighted reduction.
+        factor above 17, else rocFFT), then the weighted reduction.
         """
         buf = np.zeros(6)
         _lib.lib().aak_get_timings(self._h, _lib.dptr(buf), 6)

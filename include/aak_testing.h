@@ -55,6 +55,10 @@ int aak_test_circular_energies(const double *orbits, int n, double *E);
  * Returns their number or < 0. */
 int aak_test_eccentric(double p, double e, double cosi, double a, double dt, int maxsteps, double *out);
 
+/* Transform of the inner-product stage at a length: 0 rocFFT, 1 the fused
+ * four-step FFT, 2 the convolution; its factors R x C (optional, 0 for rocFFT). */
+int aak_test_transform(int length, int *R, int *C);
+
 /* The inner-product stage alone on two given real series of length `length`
  * (the handle's data and weights from aak_input_data): like[0..1] =
  * (<h|d>, <h|h>) as aak_Likelihood returns them, spec (optional) =
