@@ -547,11 +547,12 @@ __device__ __forceinline__ void add_bin(double2 W, double2 zk, double2 zm, doubl
   dh += x.x * d.x + x.y * d.y;
   hh += x.x * x.x + x.y * x.y;
 }
-// Bins 0 and M, both real: H_0 = E_0 + O_0, H_M = E_0 - O_0.
+// Bins 0 and M, both real: H_0 = E_0 + O_0, H_M = E_0 - O_0.  The products with
+// the zero imaginary parts stay: they pass on data that are not finite.
 __device__ __forceinline__ void add_ends(double2 z0, double2 d0, double w0, double2 dm, double wm, double &dh,
                                          double &hh) {
   const double x0 = (z0.x + z0.y) * w0, xm = (z0.x - z0.y) * wm;
-  dh += x0 * d0.x + xm * dm.x;
+  dh += x0 * d0.x + 0.0 * d0.y + xm * dm.x + 0.0 * dm.y;
   hh += x0 * x0 + xm * xm;
 }
 
