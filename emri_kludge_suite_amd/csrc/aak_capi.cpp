@@ -598,13 +598,17 @@ static int enqueue_waveform(aak_handle h, Lane &L, const DenseParams &Pplan, con
     have_deferred = defer;
     deferred_pass = pass;
   }
-  launch_fold_fill(P, B, L.stream);
-  h->mark(L, 2);
   if (Pover) {  // dense stage only
+    launch_fold_fill(P, B, L.stream);
+    h->mark(L, 2);
     HIPCHK(hipGetLastError());
     return 0;
   }
+  h->mark(L, 2);
   launch_modesum(P, B, have_deferred ? &deferred : nullptr, &fws[deferred_pass], L.stream);
+  // the tail takes the phases at the plunge as a deferred replay leaves them;
+  // the mode sum ends before it
+  launch_fold_fill(P, B, L.stream);
   h->mark(L, 3);
   HIPCHK(hipGetLastError());
   return 0;
