@@ -66,6 +66,7 @@ def lib():
         "aak_test_inspiral_rates": (_i, [_d, _d, _d, _d, _pd]),
         "aak_test_circular_energies": (_i, [_pd, _i, _pd]),
         "aak_test_eccentric": (_i, [_d, _d, _d, _d, _d, _i, _pd]),
+        "aak_test_mlp_no_pinned": (_i, [C.c_void_p, _i]),
         "aak_test_get_dense": (_i, [C.c_void_p, _pd]),
         "aak_test_transform": (_i, [_i, _pi, _pi]),
         "aak_test_inner_product": (_i, [C.c_void_p, _pd, _pd, _pd, _pd, _pi]),

@@ -527,6 +527,7 @@ struct aak_mlp_s {
   int *idx = nullptr;
   int data_n = 0;
   float *pin = nullptr;  // pinned: X | T of up to kPinRows rows, gradient, loss partials
+  bool no_pin = false;   // test hook: as if pinned memory were not to be had
   // inference scratch
   std::mutex mu;
   int icap = 0;
@@ -552,6 +553,18 @@ static void free_scratch(aak_mlp_s *m) {
 // with two uploads and two downloads, 46 against 121 at 64, 83 against 120 at
 // 16384.  Longer calls upload, so the buffer stays at 0.6 MB.
 constexpr int kPinRows = 16384;
+
+// The model's pinned buffer, formed on first use; null where it cannot be had
+// (the call then uploads).
+static float *pinned_buffer(aak_mlp_s *m) {
+  if (m->no_pin) return nullptr;
+  if (!m->pin && hipHostMalloc((void **)&m->pin, sizeof(float) * (7 * (size_t)kPinRows + kNP + kGradGroups),
+                               hipHostMallocDefault) != hipSuccess) {
+    m->pin = nullptr;
+    (void)hipGetLastError();
+  }
+  return m->pin;
+}
 
 static int grad_groups(int B) { return std::min(kGradGroups, (B + GROWS - 1) / GROWS); }
 
@@ -764,14 +777,11 @@ int aak_mlp_forward(aak_mlp m, const float *X, int n, float *Y) {
 int aak_mlp_gradient(aak_mlp m, const float *X, const float *T, int n, float *grad, double *loss) {
   if (!m || !X || !T || !grad || n <= 0) return fail(-2, "bad argument");
   MLPCHK(hipSetDevice(m->dev));
-  if (n <= kPinRows) {
+  if (n <= kPinRows && pinned_buffer(m)) {
     // the kernels read the rows from pinned host memory, each once, and leave
     // the gradient there
     int rc = grow_scratch(m, n, 0);
     if (rc) return rc;
-    if (!m->pin)
-      MLPCHK(hipHostMalloc((void **)&m->pin, sizeof(float) * (7 * (size_t)kPinRows + kNP + kGradGroups),
-                           hipHostMallocDefault));
     float *pX = m->pin, *pT = pX + 4 * (size_t)kPinRows, *pG = pT + 3 * (size_t)kPinRows, *pL = pG + kNP;
     std::memcpy(pX, X, sizeof(float) * 4 * (size_t)n);
     std::memcpy(pT, T, sizeof(float) * 3 * (size_t)n);
@@ -794,6 +804,12 @@ int aak_mlp_gradient(aak_mlp m, const float *X, const float *T, int n, float *gr
   MLPCHK(hipMemcpyAsync(grad, m->grad, sizeof(float) * kNP, hipMemcpyDeviceToHost, m->s));
   MLPCHK(hipStreamSynchronize(m->s));
   if (loss) *loss = ls / (3.0 * n);
+  return 0;
+}
+
+int aak_test_mlp_no_pinned(aak_mlp m, int on) {
+  if (!m) return fail(-1, "null model");
+  m->no_pin = on != 0;
   return 0;
 }
 

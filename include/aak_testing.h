@@ -89,6 +89,11 @@ int aak_test_fold_mode(struct aak_handle_s *h, int mode);
  * rate is rewritten in place; returns the number of replaced samples. */
 int aak_test_phidot_guard(double *rate, int n, int i0, int guard_last);
 
+/* on = 1: later gradients of the model go as where no pinned memory is to be
+ * had (their rows are uploaded).  0: off. */
+struct aak_mlp_s;
+int aak_test_mlp_no_pinned(struct aak_mlp_s *m, int on);
+
 /* Copies the dense arrays of the last aak_gpu_gen_AAK to the host:
  * out[10*(length+1)] = e | v | M | S | gimdot | Phidot | alpdot | gim | Phi | alp. */
 int aak_test_get_dense(struct aak_handle_s *h, double *out);
