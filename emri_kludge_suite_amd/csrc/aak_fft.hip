@@ -1010,7 +1010,7 @@ void launch_fft_final_reset(double *partials, int npairs, hipStream_t s) {
   hipLaunchKernelGGL(k_fft_final_reset, dim3(8), dim3(256), 0, s, partials, 2 * npairs);
 }
 
-// ---------------------------------------------------------------- other lengths
+// ------------------------------------------- data and weights in bin order
 template <int LC>
 static void launch_natural(const FftArgs &F, const double2 *Y, double *partials, hipStream_t s) {
   hipLaunchKernelGGL(k_fft_rows_natural<LC>, dim3(F.R / (2 * kNatRows), 2), dim3(2 * kNatRows * fft_threads<LC>()), 0,
@@ -1047,6 +1047,7 @@ bool launch_fft_small(const FftArgs &F, const double *h0, const double *h1, doub
   return true;
 }
 
+// ---------------------------------------------------------------- other lengths
 // Columns of 2^a points, rows of 2^a, 3 2^a or 9 2^a.
 static const int kChirpRows[] = {16,  32,  48,  64,  96,  128, 144,  192,  256, 288,
                                  384, 512, 576, 768, 1024, 1152, 1536, 2048, 2304};

@@ -6,14 +6,15 @@
 //   fold kernels   the Adams-Bashforth phase folds (AAK.cc:244-293) computed in
 //                  parallel but reproducing the sequential FP64 rounding bit for
 //                  bit: inside one binade every value is an integer multiple of
-//                  the same ulp, so the fold becomes an exact int64 prefix sum;
-//                  binade crossings, exact ties and values near zero are
-//                  replayed serially in FP64
+//                  the same ulp, so sums of the rounded steps are exact: FP64
+//                  scans in the single pass (k_fold_resolve), int64 prefix sums
+//                  in the three-pass form; binade crossings and values near
+//                  zero are replayed serially in FP64, exact ties by parity
 //   k_modesum      harmonic sum with Bessel amplitudes, Doppler phases, LISA
-//                  response and Planck taper (AAK.cc:409-547): per 256-sample
-//                  block the amplitudes are Taylor-expanded in e
-//                  (k_modesum_setup); blocks where that does not apply are
-//                  summed per sample (k_modesum_direct)
+//                  response and Planck taper (AAK.cc:409-547): per block of 1024
+//                  or 256 samples the amplitudes are Taylor-expanded in e
+//                  (k_modesum_setup); 256-sample blocks where that does not
+//                  apply are summed per sample (k_modesum_direct)
 //   k_weighted_dot PSD-weighted inner products of a rocFFT spectrum (lengths
 //                  the fused FFT of aak_fft.hip does not take), k_dot_final
 //                  the last reduction of either form (AAK_manager.cu:352-446)
@@ -119,7 +120,8 @@ __host__ __device__ inline int rates_last(const DenseParams &P) {
 // the terms in cos(iota) alone; quotients by one divisor share its reciprocal,
 // 12 divisions for the price of 7.  With 128 registers four workgroups fit a
 // CU, so the grid is cut into at most 1024 equal parts (a 1025th would run
-// alone after them).  At N = 2^21 the stage, with the guard, takes 51 us: 60 with
+// alone after them), more only where the knots in LDS or 64 samples per thread
+// limit a part.  At N = 2^21 the stage, with the guard, takes 51 us: 60 with
 // one sample per thread and separate divisions, 53 with 4 per thread in 2050
 // workgroups, 72 with five workgroups per CU (96 registers, spills).  Below
 // 2^18 samples each thread takes one, as before: 20 us at 2^17 either way, 24
@@ -2690,7 +2692,8 @@ __global__ __launch_bounds__(kMsThreads) void k_modesum_direct(DenseParams P, De
   }
 }
 
-// Workgroups of k_modesum the device runs at once (CUs x occupancy), per precision.
+// Setup (every wave of an expansion block, and the replay of a deferred fold),
+// the sum, and the blocks left to the per-sample path.
 void launch_modesum(const DenseParams &P, const DenseBuffers &B, const FoldArgs *replay, const FoldWork *fw,
                     hipStream_t s) {
   const int nb = modesum_blocks(P), ne = expansion_blocks(P);

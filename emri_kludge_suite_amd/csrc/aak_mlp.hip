@@ -215,7 +215,7 @@ __device__ __forceinline__ void load_frags(Frags f, const uint16_t *W, int l, in
 #pragma unroll
     for (int k = 0; k < 4; k++) f[t][k] = load8(W + (col0 + 16 * t + (l & 15)) * H + 32 * k + 8 * (l >> 4));
 }
-// acc[t] = (16 rows of act) x (the four column blocks of f)
+// acc[t] = (16 rows of act) x (the wave's column blocks, f)
 __device__ __forceinline__ void frag_gemm(floatx4 acc[CB], const uint16_t *act, const Frags f, int l) {
 #pragma unroll
   for (int t = 0; t < CB; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};

@@ -184,7 +184,8 @@ class GPUAAK:
     def set_tuning(self, feed_depth=-1, exp_shift=-1):
         """Batch pipeline knobs: short host plans kept ready for the GPU
         (1..256), mode-sum expansion blocks of 256 << exp_shift samples (0..3;
-        -2 restores the precision's default); < 0 (-1) keeps a knob."""
+        -2 restores the default: 2 in the mixed form and in FP64 from 2^18
+        signal samples on, else 0); < 0 (-1) keeps a knob."""
         _lib.check(_lib.lib().aak_set_tuning(self._h, int(feed_depth), int(exp_shift)), "set_tuning")
 
     def set_map_init(self, mode, model=None):
